@@ -9,8 +9,9 @@
 // windows (causal = (-1, 0), candle-core/src/accel/attention.rs:80-92), bf16 in / out, f32
 // accumulation; rows with no visible key give zeros.
 //
-// Kernel shape (head dim D = 128 or 64; one workgroup = 8 wavefronts = 64 queries x 4 query heads
-// sharing a kv head, 32 queries per wavefront):
+// Kernel shape (head dim D = 128 or 64; one workgroup = 8 wavefronts of 32 columns, a column being
+// one (query, query head) pair of a kv head, query-major: 256 columns are 64 queries of a GQA group
+// of 4, 256 of plain multi-head attention, 32 of a group of 8):
 //  * Both products run on v_mfma_f32_32x32x16_bf16. S^T = K Q^T: K (32 keys x 16 dims) comes
 //    from LDS with ds_read_b128, Q^T (pre-scaled by scale * log2(e), rounded to bf16) stays in
 //    registers for the whole key loop. The S^T accumulator of a lane holds one query column, so
@@ -42,7 +43,6 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 constexpr int kPfD = 128;          // head dim of the fused FP8 append and the E4M3 K / V path
-constexpr int kPfBQ = 64;          // queries per workgroup (two wavefronts of 32 per head)
 constexpr int kPfBK = 64;          // keys per tile of the pre-pass and of the attention at D <= 128
 
 struct PrefillArgs {
@@ -58,7 +58,7 @@ struct PrefillArgs {
     uint8_t *kc, *ks, *vc, *vs;
     uint32_t kc_plane, ks_plane, vc_plane, vs_plane;
     int32_t append, position;
-    int32_t q_len, kv_len, q_heads, kv_heads, group, heads_per_wg, q_blocks, batch;
+    int32_t q_len, kv_len, q_heads, kv_heads, group, q_blocks, batch;
     int32_t wl, wr;
     float scale_log2;
     // score terms (candle-core/kernels/flash_attn_impl.h:42-47, fa_logit), in the exp2 units of
@@ -157,9 +157,9 @@ __device__ inline int swz_vt(int d) {
     else return (d >> 2) & 3;
 }
 // Per head dim:
-//  * the workgroup: W wavefronts, W / 2 query heads x 2 halves of the 64 queries (8 at D <= 128,
-//    two per SIMD; 4 at D = 256, one per SIMD with VGPRs and AGPRs, as the 32 x 256 accumulator,
-//    the queries and the scores take more than 256 registers);
+//  * the workgroup: W wavefronts of 32 columns, NC columns in all (8 at D <= 128, two per SIMD; 4
+//    at D = 256, one per SIMD with VGPRs and AGPRs, as the 32 x 256 accumulator, the queries and
+//    the scores take more than 256 registers);
 //  * key tiles of BK keys (64; 32 at D = 256, so that four ring stages of K and V^T fit in LDS):
 //    MB 32-key blocks of S, KK 16-key steps of O^T += V^T P^T;
 //  * 16-dim k-steps of S = K Q^T, 32-dim blocks of O^T, bytes of a K row and tile, of a V^T row
@@ -171,7 +171,7 @@ __device__ inline int swz_vt(int d) {
 //    conversions; then row sums, shift and row maximum).
 template <int D>
 struct PfGeom {
-    static constexpr int W = D == 256 ? 4 : 8;
+    static constexpr int W = D == 256 ? 4 : 8, NC = 32 * W;
     static constexpr int BK = D == 256 ? 32 : 64, MB = BK / 32, KK = BK / 16, VTROW = 2 * BK;
     static constexpr int KS = D / 16, MD = D / 32;
     static constexpr int ROW = 2 * D, KTILE = BK * ROW, VTILE = D * VTROW;
@@ -255,7 +255,7 @@ PF_INLINE void pf_copy_offsets(uint32_t *koff, uint32_t *voff, int64_t k_st, int
 
 template <int D>
 struct PfState {
-    u32x4 qop[D / 16];  // Q^T operands (16-dim steps ks) of this wavefront's 32 queries, raw bits
+    u32x4 qop[D / 16];  // Q^T operands (16-dim steps ks) of this wavefront's 32 columns, raw bits
     f32x16 acc[D / 32]; // O^T: 32-dim block md
     float negm;      // -m_run (0 before the first key), added to the raw scores
     f32x16 negv;     // negm in every register: the initial value of the score products when
@@ -349,7 +349,8 @@ PF_INLINE void pf_qk(f32x16 *s, const PfState<D> &st, const uint8_t *k_lds, cons
 struct PfLogit {
     float cap2;   // softcap * log2(e) (0: off)
     float e2;     // 2 log2(e) / cap2: exp2(s * e2) = e^(2 s / cap2)
-    float slope2; // ALiBi slope * log2(e) of the wavefront's head (0: off)
+    float slope2; // ALiBi slope * log2(e) of the lane's head
+    int alibi;    // slopes given
     int pos;
 };
 // cap * tanh(x / cap) = cap - 2 cap / (e^(2x / cap) + 1): one exp2 and one reciprocal, exact
@@ -366,7 +367,7 @@ PF_INLINE void pf_logit(f32x16 *s, const PfLogit &lg, int k0, int lane) {
                 s[mb][j] = lg.cap2 - two_cap * __builtin_amdgcn_rcpf(e + 1.0f);
             }
     }
-    if (lg.slope2 != 0.0f) {
+    if (lg.alibi) {
         const int d0 = lg.pos - (k0 + 4 * (lane >> 5));  // pos - key of register 0
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
@@ -623,38 +624,47 @@ __global__ __launch_bounds__(PfGeom<D>::W * 64, 1) void prefill_kernel(PrefillAr
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int qr = lane & 31, h = lane >> 5;
 
-    // 1-D grid: consecutive workgroup ids walk the planes (batch, kv head, head group) first, so
-    // the workgroups of one plane share an XCD (ids are dealt round-robin to the 8 XCDs) and its
-    // L2; the query blocks with the most key tiles come first.
-    // head groups of up to heads_per_wg heads; the last one of a group that is not a multiple
-    // (e.g. 7 = 4 + 3 for 28 / 4 heads) leaves its spare wavefronts idle
-    const int hgroups = (a.group + a.heads_per_wg - 1) / a.heads_per_wg;
-    const int nplanes = a.kv_heads * hgroups * a.batch;
+    // 1-D grid: consecutive workgroup ids walk the planes (batch, kv head) first, so the workgroups
+    // of one plane share an XCD (ids are dealt round-robin to the 8 XCDs) and its L2; the column
+    // blocks with the most key tiles come first.
+    // Columns of a plane are (query, head of the group) pairs, query-major: column c is query
+    // c / group, head c % group, so every wavefront is full whatever the group. With 32 queries of
+    // one head per wavefront and 4 heads of 64 queries per workgroup, a group of 1 left 6 of the 8
+    // wavefronts idle (9 sequences of up to 1900 tokens, 16 / 16 heads, D = 64, f16: 195 -> 83 us
+    // per call; groups of 4 and 8 measured the same both ways).
+    const int nplanes = a.kv_heads * a.batch;
     const int plane = (int)blockIdx.x % nplanes;
     const int qb = a.q_blocks - 1 - (int)blockIdx.x / nplanes;
-    const int b = plane / (a.kv_heads * hgroups);
-    const int rem = plane % (a.kv_heads * hgroups);
-    const int hk = rem % a.kv_heads, hgrp = rem / a.kv_heads;
-    const int hslot = wave % (G::W / 2), qhalf = wave / (G::W / 2);
-    const int head = hk * a.group + hgrp * a.heads_per_wg + hslot;
-    const bool wave_live = hslot < a.heads_per_wg && hgrp * a.heads_per_wg + hslot < a.group;
-    const int q0 = qb * kPfBQ;
+    const int b = plane / a.kv_heads, hk = plane % a.kv_heads;
     const PfSeq sq = pf_sequence(a, b);
     const int lq = sq.lq, lk = sq.lk;
-    if (q0 >= lq) return;  // a shorter sequence of a variable-length batch: the whole workgroup
+    const int64_t ncols = (int64_t)lq * a.group, c0 = (int64_t)qb * G::NC;
+    if (c0 >= ncols) return;  // a shorter sequence of a variable-length batch: the whole workgroup
+    const int q0 = (int)(c0 / a.group);              // the first column's query
+    const int cr0 = (int)(c0 - (int64_t)q0 * a.group);  // and its place in the group
+    const int ncol = (int)min((int64_t)G::NC, ncols - c0);
 
-    int lo_first, hi_first, lo_last, hi_last;
-    pf_key_range(q0, lq, lk, a.wl, a.wr, lo_first, hi_first);
-    pf_key_range(min(q0 + kPfBQ, lq) - 1, lq, lk, a.wl, a.wr, lo_last, hi_last);
-    const int kt_begin = lo_first / G::BK;
-    const int ntiles = (hi_last + G::BK - 1) / G::BK - kt_begin;
+    // the workgroup's key tiles: from the first query's first visible key to the last query's last
+    int lo, hi;
+    pf_key_range(q0, lq, lk, a.wl, a.wr, lo, hi);
+    const int kt_begin = lo / G::BK;
+    pf_key_range(q0 + (cr0 + ncol - 1) / a.group, lq, lk, a.wl, a.wr, lo, hi);
+    const int ntiles = (hi + G::BK - 1) / G::BK - kt_begin;
+    // this wavefront's: it is done after the last visible key of its own last query, and then only
+    // keeps up the copies and barriers (none of its own when its columns lie past the end)
+    const bool wave_live = 32 * wave < ncol;
+    int lo_last, hi_first;
+    pf_key_range(q0 + (cr0 + min(32 * wave, ncol - 1)) / a.group, lq, lk, a.wl, a.wr, lo, hi_first);
+    pf_key_range(q0 + (cr0 + min(32 * wave + 32, ncol) - 1) / a.group, lq, lk, a.wl, a.wr, lo_last, hi);
+    const int wtiles = wave_live ? max((hi + G::BK - 1) / G::BK - kt_begin, 0) : 0;
 
     PfState<D> st;
     {
-        const int qi = q0 + 32 * qhalf + qr;
-        const bool ok = wave_live && qi < lq;
-        const uint16_t *row = a.q + sq.q0 + (int64_t)min(head, a.q_heads - 1) * a.q_sh +
-                              (int64_t)min(qi, lq - 1) * a.q_st;
+        const bool ok = 32 * wave + qr < ncol;
+        const int c = cr0 + min(32 * wave + qr, ncol - 1);
+        const int qi = q0 + c / a.group;
+        const uint16_t *row = a.q + sq.q0 + (int64_t)(hk * a.group + c % a.group) * a.q_sh +
+                              (int64_t)qi * a.q_st;
         const float qs = a.scale_log2 * a.q_mul * (a.q_mul_dev ? a.q_mul_dev[0] : 1.0f);
         // (QRAW: a zero factor is made the smallest normal one, so masked scores stay -inf)
         st.c2 = qs == 0.0f ? 1.17549435e-38f : qs;
@@ -674,7 +684,7 @@ __global__ __launch_bounds__(PfGeom<D>::W * 64, 1) void prefill_kernel(PrefillAr
             }
             st.qop[ks] = w;
         }
-        if (qi < lq) pf_key_range(qi, lq, lk, a.wl, a.wr, st.qlo, st.qhi);
+        if (ok) pf_key_range(qi, lq, lk, a.wl, a.wr, st.qlo, st.qhi);
         else st.qlo = st.qhi = 0;
         st.m_run = -__builtin_inff();
         st.thr = -__builtin_inff();
@@ -691,8 +701,10 @@ __global__ __launch_bounds__(PfGeom<D>::W * 64, 1) void prefill_kernel(PrefillAr
     if (LOGIT) {
         lg.cap2 = a.softcap2;
         lg.e2 = a.softcap2 > 0.0f ? 2.0f * kLog2e / a.softcap2 : 0.0f;
-        lg.slope2 = a.alibi && wave_live ? a.alibi[(int64_t)b * a.alibi_bs + head] * kLog2e : 0.0f;
-        lg.pos = q0 + 32 * qhalf + qr + lk - lq;
+        const int c = cr0 + min(32 * wave + qr, ncol - 1);
+        lg.alibi = a.alibi != nullptr;
+        lg.slope2 = a.alibi ? a.alibi[(int64_t)b * a.alibi_bs + hk * a.group + c % a.group] * kLog2e : 0.0f;
+        lg.pos = q0 + c / a.group + lk - lq;
     }
     PF_WAIT_VMCNT(0);  // the Q loads above must not be counted by the copy waits below
 
@@ -724,17 +736,6 @@ __global__ __launch_bounds__(PfGeom<D>::W * 64, 1) void prefill_kernel(PrefillAr
         PF_WAIT_VMCNT(G::CP);                                                                \
         __builtin_amdgcn_s_barrier();                                                        \
     }
-    if (!wave_live) {  // heads past the group: copies and barriers only
-        for (int t = 0; t < ntiles;) {
-            PF_SYNC(0, t) PF_ISSUE(3, t + 3); if (++t == ntiles) break;
-            PF_SYNC(1, t) PF_ISSUE(0, t + 3); if (++t == ntiles) break;
-            PF_SYNC(2, t) PF_ISSUE(1, t + 3); if (++t == ntiles) break;
-            PF_SYNC(3, t) PF_ISSUE(2, t + 3); ++t;
-        }
-        PF_WAIT_VMCNT(0);
-        return;
-    }
-
     const auto tile_masked = [&](int kt) {
         const int k0 = (kt_begin + kt) * G::BK;
         return !(k0 >= lo_last && k0 + G::BK <= hi_first);
@@ -743,7 +744,7 @@ __global__ __launch_bounds__(PfGeom<D>::W * 64, 1) void prefill_kernel(PrefillAr
     u32x4 pop[2 * G::MB];
     PfAddr<D> ad;
     pf_addr_init<D>(ad, lane);
-    if (ntiles > 0) {
+    if (wtiles > 0) {
         pf_qk<F16, D>(sa, st, ks0, ad, f32x16{});  // (negm is 0 here)
         if (LOGIT) {
             if constexpr (G::QRAW) pf_scale<G::MB>(sa, st.c2);
@@ -757,13 +758,13 @@ __global__ __launch_bounds__(PfGeom<D>::W * 64, 1) void prefill_kernel(PrefillAr
         if (__any(need)) pf_rescale(sa, st, mx, need);
     }
     // Step t: S(t) in CUR, stage t % 4 holds V(t), stage (t + 1) % 4 holds K(t + 1); the
-    // copies of tile t + 3 go into stage (t + 3) % 4 in block 2. The last tile leaves the loop
-    // (its stage in `last`) and is finished after it.
+    // copies of tile t + 3 go into stage (t + 3) % 4 in block 2. The wavefront's last tile leaves
+    // the loop (its stage in `last`) and is finished after it.
 #define PF_STEP(k, CUR, NXT)                                                                 \
     {                                                                                        \
         pf_addr_opaque(ad);                                                                  \
         PF_SYNC(k, t)                                                                        \
-        if (t + 1 == ntiles) {                                                               \
+        if (t + 1 == wtiles) {                                                               \
             last = k;                                                                        \
             break;                                                                           \
         }                                                                                    \
@@ -774,22 +775,36 @@ __global__ __launch_bounds__(PfGeom<D>::W * 64, 1) void prefill_kernel(PrefillAr
         ++t;                                                                                 \
     }
     int last = 0;
-    if (ntiles > 0) {
+    if (wtiles > 0) {
         for (int t = 0;;) {
             PF_STEP(0, sa, sb)
             PF_STEP(1, sb, sa)
             PF_STEP(2, sa, sb)
             PF_STEP(3, sb, sa)
         }
-        PF_WAIT_VMCNT(0);  // the dummy copies past the end
         pf_addr_opaque(ad);
         switch (last) {
-            case 0: pf_last_tile<F16, D>(sa, pop, st, vs0, ad); break;
-            case 1: pf_last_tile<F16, D>(sb, pop, st, vs1, ad); break;
-            case 2: pf_last_tile<F16, D>(sa, pop, st, vs2, ad); break;
-            default: pf_last_tile<F16, D>(sb, pop, st, vs3, ad); break;
+            case 0: PF_ISSUE(3, wtiles + 2); pf_last_tile<F16, D>(sa, pop, st, vs0, ad); break;
+            case 1: PF_ISSUE(0, wtiles + 2); pf_last_tile<F16, D>(sb, pop, st, vs1, ad); break;
+            case 2: PF_ISSUE(1, wtiles + 2); pf_last_tile<F16, D>(sa, pop, st, vs2, ad); break;
+            default: PF_ISSUE(2, wtiles + 2); pf_last_tile<F16, D>(sb, pop, st, vs3, ad); break;
         }
     }
+    // (pinned here: every V^T read of the last tile is back before the barriers below)
+#pragma unroll
+    for (int md = 0; md < G::MD; ++md) asm volatile("" : "+v"(st.acc[md]));
+    // the tiles that later columns of the workgroup still see: copies and barriers only (this
+    // wavefront's reads of its last V^T stage are done, so the next step may refill it)
+    for (int t = wtiles; t < ntiles; ++t) {
+        PF_SYNC(0, t)
+        switch (t & 3) {
+            case 0: PF_ISSUE(3, t + 3); break;
+            case 1: PF_ISSUE(0, t + 3); break;
+            case 2: PF_ISSUE(1, t + 3); break;
+            default: PF_ISSUE(2, t + 3); break;
+        }
+    }
+    PF_WAIT_VMCNT(0);  // the dummy copies past the end
 #undef PF_STEP
 #undef PF_SYNC
 #undef PF_ISSUE
@@ -800,9 +815,10 @@ __global__ __launch_bounds__(PfGeom<D>::W * 64, 1) void prefill_kernel(PrefillAr
     const float l = pf_sum_halves(st.l_run);
     const float om = a.o_mul * (a.o_mul_dev ? a.o_mul_dev[0] : 1.0f);
     const float inv = l > 0.0f ? om / l : 0.0f;
-    const int qi = q0 + 32 * qhalf + qr;
-    if (qi >= lq) return;
-    uint16_t *orow = a.out + sq.o0 + (int64_t)qi * a.o_st + (int64_t)head * a.o_sh;
+    if (32 * wave + qr >= ncol) return;
+    const int c = cr0 + 32 * wave + qr;
+    uint16_t *orow = a.out + sq.o0 + (int64_t)(q0 + c / a.group) * a.o_st +
+                     (int64_t)(hk * a.group + c % a.group) * a.o_sh;
 #pragma unroll
     for (int md = 0; md < G::MD; ++md)
 #pragma unroll
@@ -1221,9 +1237,8 @@ int flash_attn_impl(const void *q, const int64_t q_strides[3], const void *k,
     a.q_heads = q_heads;
     a.kv_heads = kv_heads;
     a.group = q_heads / kv_heads;
-    const int hpw = head_dim == 256 ? PfGeom<256>::W / 2 : PfGeom<128>::W / 2;  // heads per workgroup
-    a.heads_per_wg = a.group < hpw ? a.group : hpw;
-    a.q_blocks = (q_len + kPfBQ - 1) / kPfBQ;
+    const int nc = head_dim == 256 ? PfGeom<256>::NC : PfGeom<128>::NC;  // columns per workgroup
+    a.q_blocks = (int)(((int64_t)q_len * a.group + nc - 1) / nc);
     a.wl = window_left;
     a.wr = window_right;
     a.scale_log2 = softmax_scale * kLog2e;
@@ -1293,7 +1308,7 @@ int flash_attn_impl(const void *q, const int64_t q_strides[3], const void *k,
     if (head_dim == 64) hipLaunchKernelGGL(prefill_stage_kernel<64>, sgrid, dim3(256), 0, st, a);
     else if (head_dim == 256) hipLaunchKernelGGL(prefill_stage_kernel<256>, sgrid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL(prefill_stage_kernel<128>, sgrid, dim3(256), 0, st, a);
-    const dim3 grid(a.q_blocks * kv_heads * ((a.group + a.heads_per_wg - 1) / a.heads_per_wg) * batch);
+    const dim3 grid(a.q_blocks * kv_heads * batch);
     const bool terms = softcap > 0.0f || alibi_slopes;
     if (head_dim == 64) pf_launch<64>(dtype == CQKV_F16, terms, grid, st, a);
     else if (head_dim == 256) pf_launch<256>(dtype == CQKV_F16, terms, grid, st, a);
