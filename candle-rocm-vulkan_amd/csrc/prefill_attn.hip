@@ -31,6 +31,7 @@
 //  * Causal work is uneven: the workgroups with the most key tiles are dispatched first.
 #include <algorithm>
 #include <type_traits>
+#include <vector>
 
 #include "cqkv_device.h"
 #include "cqkv_host.h"
@@ -84,7 +85,19 @@ struct PrefillArgs {
     int64_t k8_sb, k8_st, k8_sh, v8_sb, v8_st, v8_sh;
     uint16_t *kst;
     int32_t e4m3, f16;
+    // split key ranges (max_pieces > 1): a workgroup's key tiles in pieces of at most piece_tiles,
+    // whose partial outputs (max_pieces, batch, kv head, q_len * group, D) f32 and lse (without the
+    // D) prefill_combine_kernel merges; column blocks of one piece write the output themselves
+    int32_t piece_tiles, max_pieces;
+    float *part_o, *part_lse;
+    uint32_t group_m;  // ceil(2^32 / group) for group 2 .. 32768, else 0
 };
+
+// c / group for the columns of a workgroup (c < group + 256): one multiplication instead of a
+// division's dependent chain in the prologue (exact, as c * (group_m * group - 2^32) < 2^32).
+__device__ inline int pf_query_of(int c, const PrefillArgs &a) {
+    return a.group == 1 ? c : a.group_m ? (int)__umulhi((uint32_t)c, a.group_m) : c / a.group;
+}
 
 // First rows and lengths of sequence b. Variable-length offsets are clamped into the tensors
 // and the lengths to q_len / kv_len, so inconsistent prefix sums cannot address memory outside
@@ -129,12 +142,28 @@ using pf_op_t = typename std::conditional<F16, f16x8, bf16x8>::type;
 __device__ inline u32x4 ldg128(const uint16_t *p) { return *(const u32x4 *)p; }
 
 // visible keys [lo, hi) of query position i (bottom-right aligned)
-__device__ inline void pf_key_range(int i, int lq, int lk, int wl, int wr, int &lo, int &hi) {
+__host__ __device__ inline void pf_key_range(int i, int lq, int lk, int wl, int wr, int &lo, int &hi) {
     const int pos = i + lk - lq;
     lo = wl >= 0 ? max(pos - wl, 0) : 0;
     hi = wr >= 0 ? min(pos + wr + 1, lk) : lk;
     lo = min(lo, lk);
     hi = max(hi, lo);
+}
+
+// Pieces that n key tiles are cut into: whole pieces of piece_tiles and a last one of up to a
+// quarter more (the rest up to a quarter is not worth a workgroup and its partials).
+__host__ __device__ inline int pf_pieces(int n, int piece_tiles, int max_pieces) {
+    const int rest = n - piece_tiles / 4;
+    return max_pieces <= 1 || rest <= piece_tiles ? 1 : min((rest + piece_tiles - 1) / piece_tiles, max_pieces);
+}
+// Key tiles (of bk keys) of the column block whose queries are q0 .. q1: first tile and count.
+__host__ __device__ inline int pf_block_tiles(int q0, int q1, int lq, int lk, int wl, int wr, int bk,
+                                              int &begin) {
+    int lo, hi, lo1;
+    pf_key_range(q0, lq, lk, wl, wr, lo, hi);
+    pf_key_range(q1, lq, lk, wl, wr, lo1, hi);
+    begin = lo / bk;
+    return max((hi + bk - 1) / bk - begin, 0);
 }
 
 // LDS K tile layout: 64 rows (keys) x 2 D bytes, no padding; the 16-byte chunk c of row r sits at
@@ -604,8 +633,9 @@ PF_INLINE void pf_last_tile(const f32x16 *cur, u32x4 *pop, PfState<D> &st,
 }
 
 // Two wavefronts per SIMD (8 per workgroup, ~240 registers each at D = 128).
-// LOGIT: soft-capping and / or ALiBi (a separate instantiation keeps them off the plain path)
-template <bool LOGIT, bool F16, int D>
+// LOGIT: soft-capping and / or ALiBi; SPLIT: max_pieces > 1 (separate instantiations keep both off
+// the plain path)
+template <bool LOGIT, bool F16, int D, bool SPLIT>
 __global__ __launch_bounds__(PfGeom<D>::W * 64, 1) void prefill_kernel(PrefillArgs a) {
     using G = PfGeom<D>;
     // the K and V^T rings: four stages each, as distinct arrays named statically below, so the
@@ -631,39 +661,55 @@ __global__ __launch_bounds__(PfGeom<D>::W * 64, 1) void prefill_kernel(PrefillAr
     // c / group, head c % group, so every wavefront is full whatever the group. With 32 queries of
     // one head per wavefront and 4 heads of 64 queries per workgroup, a group of 1 left 6 of the 8
     // wavefronts idle (9 sequences of up to 1900 tokens, 16 / 16 heads, D = 64, f16: 195 -> 83 us
-    // per call; groups of 4 and 8 measured the same both ways).
+    // per call; a group of 4 measured the same both ways).
     const int nplanes = a.kv_heads * a.batch;
-    const int plane = (int)blockIdx.x % nplanes;
-    const int qb = a.q_blocks - 1 - (int)blockIdx.x / nplanes;
+    const int rest = (int)blockIdx.x / nplanes;
+    // ragged batches whose kv heads do not cover the XCDs: the planes move on by one XCD per row of
+    // blocks, or each XCD would keep the same few sequences and the longest would end alone (12
+    // sequences of up to 2414 tokens, 32 / 2 heads, D = 64: 222 -> 189 us per call)
+    const bool turn = a.cu_q && (a.kv_heads & 7) && (nplanes & 7) == 0;
+    const int plane = (int)((blockIdx.x + (turn ? (unsigned)rest : 0u)) % (unsigned)nplanes);
+    // split key ranges: the whole pieces of every block first, then the blocks' last pieces
+    const int whole = SPLIT ? a.max_pieces - 1 : 0;
+    const bool last_piece = !SPLIT || rest >= a.q_blocks * whole;
+    const int qb = a.q_blocks - 1 - (last_piece ? rest - a.q_blocks * whole : rest / whole);
     const int b = plane / a.kv_heads, hk = plane % a.kv_heads;
     const PfSeq sq = pf_sequence(a, b);
     const int lq = sq.lq, lk = sq.lk;
     const int64_t ncols = (int64_t)lq * a.group, c0 = (int64_t)qb * G::NC;
     if (c0 >= ncols) return;  // a shorter sequence of a variable-length batch: the whole workgroup
-    const int q0 = (int)(c0 / a.group);              // the first column's query
+    const int q0 = c0 < 0x7fffffff ? (int)((uint32_t)c0 / (uint32_t)a.group)  // the first column's query
+                                   : (int)(c0 / a.group);
     const int cr0 = (int)(c0 - (int64_t)q0 * a.group);  // and its place in the group
     const int ncol = (int)min((int64_t)G::NC, ncols - c0);
 
-    // the workgroup's key tiles: from the first query's first visible key to the last query's last
-    int lo, hi;
-    pf_key_range(q0, lq, lk, a.wl, a.wr, lo, hi);
-    const int kt_begin = lo / G::BK;
-    pf_key_range(q0 + (cr0 + ncol - 1) / a.group, lq, lk, a.wl, a.wr, lo, hi);
-    const int ntiles = (hi + G::BK - 1) / G::BK - kt_begin;
+    // the workgroup's key tiles, from the first query's first visible key to the last query's last,
+    // or its piece of them
+    int kt_begin;
+    int ntiles = pf_block_tiles(q0, q0 + pf_query_of(cr0 + ncol - 1, a), lq, lk, a.wl, a.wr, G::BK,
+                                kt_begin);
+    const int pieces = SPLIT ? pf_pieces(ntiles, a.piece_tiles, a.max_pieces) : 1;
+    const int piece = last_piece ? pieces - 1 : rest % whole;
+    if (SPLIT && pieces > 1) {
+        const int first = piece * a.piece_tiles;
+        kt_begin += first;
+        ntiles = last_piece ? ntiles - first : a.piece_tiles;
+    }
+    if (piece >= pieces - (last_piece ? 0 : 1)) return;
     // this wavefront's: it is done after the last visible key of its own last query, and then only
     // keeps up the copies and barriers (none of its own when its columns lie past the end)
     const bool wave_live = 32 * wave < ncol;
-    int lo_last, hi_first;
-    pf_key_range(q0 + (cr0 + min(32 * wave, ncol - 1)) / a.group, lq, lk, a.wl, a.wr, lo, hi_first);
-    pf_key_range(q0 + (cr0 + min(32 * wave + 32, ncol) - 1) / a.group, lq, lk, a.wl, a.wr, lo_last, hi);
-    const int wtiles = wave_live ? max((hi + G::BK - 1) / G::BK - kt_begin, 0) : 0;
+    int lo, hi, lo_last, hi_first;
+    pf_key_range(q0 + pf_query_of(cr0 + min(32 * wave, ncol - 1), a), lq, lk, a.wl, a.wr, lo, hi_first);
+    pf_key_range(q0 + pf_query_of(cr0 + min(32 * wave + 32, ncol) - 1, a), lq, lk, a.wl, a.wr, lo_last, hi);
+    const int wtiles = wave_live ? min(max((hi + G::BK - 1) / G::BK - kt_begin, 0), ntiles) : 0;
 
     PfState<D> st;
     {
         const bool ok = 32 * wave + qr < ncol;
         const int c = cr0 + min(32 * wave + qr, ncol - 1);
-        const int qi = q0 + c / a.group;
-        const uint16_t *row = a.q + sq.q0 + (int64_t)(hk * a.group + c % a.group) * a.q_sh +
+        const int qc = pf_query_of(c, a), qi = q0 + qc;
+        const uint16_t *row = a.q + sq.q0 + (int64_t)(hk * a.group + (c - qc * a.group)) * a.q_sh +
                               (int64_t)qi * a.q_st;
         const float qs = a.scale_log2 * a.q_mul * (a.q_mul_dev ? a.q_mul_dev[0] : 1.0f);
         // (QRAW: a zero factor is made the smallest normal one, so masked scores stay -inf)
@@ -703,8 +749,9 @@ __global__ __launch_bounds__(PfGeom<D>::W * 64, 1) void prefill_kernel(PrefillAr
         lg.e2 = a.softcap2 > 0.0f ? 2.0f * kLog2e / a.softcap2 : 0.0f;
         const int c = cr0 + min(32 * wave + qr, ncol - 1);
         lg.alibi = a.alibi != nullptr;
-        lg.slope2 = a.alibi ? a.alibi[(int64_t)b * a.alibi_bs + hk * a.group + c % a.group] * kLog2e : 0.0f;
-        lg.pos = q0 + c / a.group + lk - lq;
+        const int qc = pf_query_of(c, a), head = hk * a.group + (c - qc * a.group);
+        lg.slope2 = a.alibi ? a.alibi[(int64_t)b * a.alibi_bs + head] * kLog2e : 0.0f;
+        lg.pos = q0 + qc + lk - lq;
     }
     PF_WAIT_VMCNT(0);  // the Q loads above must not be counted by the copy waits below
 
@@ -816,9 +863,24 @@ __global__ __launch_bounds__(PfGeom<D>::W * 64, 1) void prefill_kernel(PrefillAr
     const float om = a.o_mul * (a.o_mul_dev ? a.o_mul_dev[0] : 1.0f);
     const float inv = l > 0.0f ? om / l : 0.0f;
     if (32 * wave + qr >= ncol) return;
-    const int c = cr0 + 32 * wave + qr;
-    uint16_t *orow = a.out + sq.o0 + (int64_t)(q0 + c / a.group) * a.o_st +
-                     (int64_t)(hk * a.group + c % a.group) * a.o_sh;
+    if (SPLIT && pieces > 1) {  // this piece's normalised rows and their log2-sum-exp, f32
+        const float invl = l > 0.0f ? 1.0f / l : 0.0f;
+        const int64_t row = ((int64_t)piece * nplanes + plane) * ((int64_t)a.q_len * a.group) +
+                            (c0 + 32 * wave + qr);
+        if (h == 0) a.part_lse[row] = l > 0.0f ? st.m_run + __builtin_amdgcn_logf(l) : -__builtin_inff();
+        float *po = a.part_o + row * D + 4 * h;
+#pragma unroll
+        for (int md = 0; md < G::MD; ++md)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                *(f32x4 *)(po + 32 * md + 8 * j) =
+                    f32x4{st.acc[md][4 * j] * invl, st.acc[md][4 * j + 1] * invl,
+                          st.acc[md][4 * j + 2] * invl, st.acc[md][4 * j + 3] * invl};
+        return;
+    }
+    const int c = cr0 + 32 * wave + qr, qc = pf_query_of(c, a);
+    uint16_t *orow = a.out + sq.o0 + (int64_t)(q0 + qc) * a.o_st +
+                     (int64_t)(hk * a.group + (c - qc * a.group)) * a.o_sh;
 #pragma unroll
     for (int md = 0; md < G::MD; ++md)
 #pragma unroll
@@ -833,6 +895,68 @@ __global__ __launch_bounds__(PfGeom<D>::W * 64, 1) void prefill_kernel(PrefillAr
             }
             *(u32x2 *)(orow + 32 * md + 8 * j + 4 * h) = w;
         }
+}
+
+// Merges the pieces of the column blocks that have more than one: o = sum_p w_p o_p / sum_p w_p with
+// w_p = 2^(lse_p - max lse) (tq_combine_impl's formula, candle-core/kernels/turbo_quant_impl.h:
+// 659-685), pieces without a visible key skipped. D / 4 lanes per column, 4 head dims each; lane p of
+// each 16 loads piece p's lse (at most kPfMaxPieces = 16), so the weights cost one load's latency.
+constexpr int kPfMaxPieces = 16;
+template <bool F16, int D>
+__global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a) {
+    using G = PfGeom<D>;
+    constexpr int L = D / 4;  // lanes per column
+    static_assert(L % kPfMaxPieces == 0, "whole groups of one lane per piece");
+    const int li = threadIdx.x % L;
+    const int plane = blockIdx.y;
+    const int b = plane / a.kv_heads, hk = plane % a.kv_heads;
+    const int64_t col = (int64_t)blockIdx.x * (256 / L) + threadIdx.x / L;
+    const PfSeq sq = pf_sequence(a, b);
+    const int64_t ncols = (int64_t)sq.lq * a.group;
+    if (col >= ncols) return;
+    const int64_t c0 = col / G::NC * G::NC;
+    int begin;
+    const int n = pf_block_tiles((int)(c0 / a.group), (int)((min(c0 + G::NC, ncols) - 1) / a.group),
+                                 sq.lq, sq.lk, a.wl, a.wr, G::BK, begin);
+    const int pieces = pf_pieces(n, a.piece_tiles, a.max_pieces);
+    if (pieces <= 1) return;
+    const int64_t rows = (int64_t)a.q_len * a.group;  // of a plane
+    const int64_t step = rows * a.kv_heads * a.batch;
+    const int64_t row = plane * rows + col;
+    const int pl = li % kPfMaxPieces;
+    const float e = pl < pieces ? a.part_lse[row + pl * step] : -__builtin_inff();
+    float M = e;
+#pragma unroll
+    for (int o = 1; o < kPfMaxPieces; o <<= 1) M = fmaxf(M, __shfl_xor(M, o, kPfMaxPieces));
+    const float w = e == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(e - M);
+    float sum = w;
+#pragma unroll
+    for (int o = 1; o < kPfMaxPieces; o <<= 1) sum += __shfl_xor(sum, o, kPfMaxPieces);
+    const float *po = a.part_o + row * D + 4 * li;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int p0 = 0; p0 < pieces; p0 += 4) {  // four pieces' rows in flight
+        f32x4 v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = *(const f32x4 *)(po + min(p0 + i, pieces - 1) * step * D);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float wp = __shfl(w, p0 + i, kPfMaxPieces);  // 0 past the last piece
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc[k] += wp > 0.0f ? wp * v[i][k] : 0.0f;
+        }
+    }
+    const float om = a.o_mul * (a.o_mul_dev ? a.o_mul_dev[0] : 1.0f);
+    const float inv = sum > 0.0f ? om / sum : 0.0f;
+    const int qi = (int)(col / a.group), g = (int)(col % a.group);
+    u32x2 r;
+    if constexpr (F16) {
+        r.x = pack_f16x2(acc[0] * inv, acc[1] * inv);
+        r.y = pack_f16x2(acc[2] * inv, acc[3] * inv);
+    } else {
+        r.x = pack_bf16x2(acc[0] * inv, acc[1] * inv);
+        r.y = pack_bf16x2(acc[2] * inv, acc[3] * inv);
+    }
+    *(u32x2 *)(a.out + sq.o0 + (int64_t)qi * a.o_st + (int64_t)(hk * a.group + g) * a.o_sh + 4 * li) = r;
 }
 
 // Pre-pass, one workgroup per 64-key tile of a (batch, kv head) plane, through LDS:
@@ -1032,6 +1156,84 @@ static size_t pf_kst_bytes(int32_t batch, int32_t kv_len, int32_t kv_heads) {
     return (size_t)batch * kv_heads * kv_len * kPfD * 2;
 }
 
+// How a call's key ranges are split: column blocks of more than `tiles` key tiles in up to `pieces`
+// pieces (1: not at all), and the bytes of the partials.
+struct PfPlan {
+    int tiles = 1 << 30, pieces = 1;
+    size_t bytes = 0;
+};
+// A CU holds one workgroup, so a call of few column blocks leaves CUs idle: one 300-token chunk of a
+// 32 / 8-head model over 7000 keys is 40 blocks of 110 tiles on 256 CUs (157 -> 54 us per call in 6
+// pieces). The count with the smallest estimate is taken:
+//  * steps: key tiles that the last CU to end works through, a workgroup costing kSetup tiles beside
+//    its own (its queries, the first tiles' latency, the output). Up to 256 workgroups: the longest;
+//    more: the mean per CU and half a workgroup.
+//  * a step takes lo us on an idle chip and up to hi us more the fuller it is (clocks, caches: at
+//    D = 128, 1.3 us with 40 workgroups, 1.86 us with 200), so t = lo * steps + hi * mean tiles per CU.
+//  * the combine: 3 us, and its partials written and read, mostly cached, at 8 TB/s (6.8 us for 9600
+//    rows of 5 pieces).
+// A causal prompt of about as many blocks as CUs keeps them whole: its mean is half of its longest,
+// but the rate rises as CUs fall idle, and the partials cost what is left (2048 tokens, 32 / 8 heads:
+// 62.6 us whole, 66.2 us in halves; 3000 tokens: 91.7 and 110.2). No piece is under 512 keys, so
+// shorter sequences are never split.
+static PfPlan pf_plan(int head_dim, int batch, int q_len, int kv_len, int q_heads, int kv_heads,
+                      int wl, int wr) {
+    constexpr int kCus = 256, kSetup = 3;
+    const int nc = head_dim == 256 ? PfGeom<256>::NC : PfGeom<128>::NC;
+    const int bk = head_dim == 256 ? PfGeom<256>::BK : PfGeom<128>::BK;
+    const int min_tiles = 512 / bk, group = q_heads / kv_heads;
+    const double lo = head_dim == 64 ? 0.76 : head_dim == 128 ? 1.2 : 0.7;
+    const double hi = head_dim == 64 ? 0.4 : head_dim == 128 ? 0.75 : 0.4;
+    const int64_t planes = (int64_t)batch * kv_heads, cols = (int64_t)q_len * group;
+    const int64_t blocks = (cols + nc - 1) / nc;
+    PfPlan best;
+    if (planes * blocks > 2 * kCus || kv_len <= 512) return best;
+    std::vector<int> n(blocks);  // key tiles, in the order the blocks are handed out
+    int most = 0;
+    for (int64_t i = 0; i < blocks; ++i) {
+        const int64_t c0 = (blocks - 1 - i) * nc;
+        int begin;
+        n[i] = pf_block_tiles((int)(c0 / group), (int)((std::min(c0 + nc, cols) - 1) / group), q_len,
+                              kv_len, wl, wr, bk, begin);
+        most = std::max(most, n[i]);
+    }
+    double best_us = 0.0;
+    for (int p = 1; p <= kPfMaxPieces; ++p) {
+        const int tiles = (most + p - 1) / p;
+        if (p > 1 && (tiles < min_tiles || planes * blocks * p > 8 * kCus)) break;
+        int64_t wgs = 0, total = 0, split_cols = 0;
+        int longest = 0;
+        for (int64_t i = 0; i < blocks; ++i) {
+            const int k = pf_pieces(n[i], tiles, p);
+            const int last = n[i] - (k - 1) * tiles;
+            longest = std::max(longest, k > 1 ? std::max(last, tiles) : last);
+            wgs += planes * k;
+            total += planes * (n[i] + (int64_t)k * kSetup);
+            if (k > 1) split_cols += k * nc;
+        }
+        const double mean = (double)total / kCus;
+        double steps = longest + kSetup;
+        if (wgs > kCus) steps = std::max(steps, mean + 0.5 * total / wgs);
+        double t = lo * steps + hi * mean;
+        if (p > 1) t += 3.0 + (double)planes * split_cols * head_dim * 8 / 8e6;
+        if (p == 1 || t < (best.pieces == 1 ? 0.92 : 0.97) * best_us) {
+            best_us = t;
+            best.tiles = tiles;
+            best.pieces = p;
+        }
+    }
+    if (best.pieces > 1)
+        best.bytes = ((size_t)best.pieces * planes * cols * head_dim * 4 + 255) / 256 * 256 +
+                     (size_t)best.pieces * planes * cols * 4;
+    return best;
+}
+// Bytes of the partials whatever the window: the larger of the causal and the full mask's plan (a
+// call whose own plan needs more than its workspace holds is not split).
+static size_t pf_part_bytes(int head_dim, int batch, int q_len, int kv_len, int q_heads, int kv_heads) {
+    return std::max(pf_plan(head_dim, batch, q_len, kv_len, q_heads, kv_heads, -1, 0).bytes,
+                    pf_plan(head_dim, batch, q_len, kv_len, q_heads, kv_heads, -1, -1).bytes);
+}
+
 bool prefill_takes(int32_t dtype, int32_t head_dim, int32_t q_len, const void *q,
                    const int64_t q_strides[3], const void *out, const int64_t out_strides[3]) {
     auto aligned = [](const void *p, const int64_t st[3], int bytes) {
@@ -1059,20 +1261,33 @@ size_t flash_attn_workspace(int32_t dtype, int32_t batch, int32_t q_len, int32_t
     // a call of the MFMA prefill's shape whose q / out rows are not aligned for it runs the
     // plain kernel: size for either
     if (kv_len > 0 && pf_fast_path(dtype, head_dim, q_len))
-        return std::max(pf_vt_bytes(batch, kv_len, kv_heads, head_dim), plain);
+        return std::max((pf_vt_bytes(batch, kv_len, kv_heads, head_dim) + 255) / 256 * 256 +
+                            pf_part_bytes(head_dim, batch, q_len, kv_len, q_heads, kv_heads),
+                        plain);
     return plain;
+}
+
+template <int D, bool SPLIT>
+static void pf_launch_kernel(bool f16, bool terms, dim3 grid, hipStream_t st, const PrefillArgs &a) {
+    const dim3 block(PfGeom<D>::W * 64);
+    if (f16) {
+        if (terms) hipLaunchKernelGGL((prefill_kernel<true, true, D, SPLIT>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((prefill_kernel<false, true, D, SPLIT>), grid, block, 0, st, a);
+    } else {
+        if (terms) hipLaunchKernelGGL((prefill_kernel<true, false, D, SPLIT>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((prefill_kernel<false, false, D, SPLIT>), grid, block, 0, st, a);
+    }
 }
 
 template <int D>
 static void pf_launch(bool f16, bool terms, dim3 grid, hipStream_t st, const PrefillArgs &a) {
-    const dim3 block(PfGeom<D>::W * 64);
-    if (f16) {
-        if (terms) hipLaunchKernelGGL((prefill_kernel<true, true, D>), grid, block, 0, st, a);
-        else hipLaunchKernelGGL((prefill_kernel<false, true, D>), grid, block, 0, st, a);
-    } else {
-        if (terms) hipLaunchKernelGGL((prefill_kernel<true, false, D>), grid, block, 0, st, a);
-        else hipLaunchKernelGGL((prefill_kernel<false, false, D>), grid, block, 0, st, a);
-    }
+    if (a.max_pieces <= 1) return pf_launch_kernel<D, false>(f16, terms, grid, st, a);
+    pf_launch_kernel<D, true>(f16, terms, grid, st, a);
+    constexpr int cpw = 256 / (D / 4);  // columns per workgroup
+    const int64_t cols = (int64_t)a.q_len * a.group;
+    const dim3 cgrid((unsigned)((cols + cpw - 1) / cpw), (unsigned)(a.kv_heads * a.batch));
+    if (f16) hipLaunchKernelGGL((prefill_combine_kernel<true, D>), cgrid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((prefill_combine_kernel<false, D>), cgrid, dim3(256), 0, st, a);
 }
 
 int flash_attn_impl(const void *q, const int64_t q_strides[3], const void *k,
@@ -1237,6 +1452,7 @@ int flash_attn_impl(const void *q, const int64_t q_strides[3], const void *k,
     a.q_heads = q_heads;
     a.kv_heads = kv_heads;
     a.group = q_heads / kv_heads;
+    a.group_m = a.group > 1 && a.group <= 32768 ? (uint32_t)(0x100000000ull / a.group + (0x100000000ull % a.group != 0)) : 0;
     const int nc = head_dim == 256 ? PfGeom<256>::NC : PfGeom<128>::NC;  // columns per workgroup
     a.q_blocks = (int)(((int64_t)q_len * a.group + nc - 1) / nc);
     a.wl = window_left;
@@ -1260,13 +1476,25 @@ int flash_attn_impl(const void *q, const int64_t q_strides[3], const void *k,
     void *vt = workspace;
     const size_t vt_bytes = pf_vt_bytes(batch, kv_len, kv_heads, head_dim);
     const size_t kst_off = (vt_bytes + 255) / 256 * 256;
-    const size_t ws_bytes = e4m3 ? kst_off + pf_kst_bytes(batch, kv_len, kv_heads) : vt_bytes;
+    size_t ws_bytes = e4m3 ? kst_off + pf_kst_bytes(batch, kv_len, kv_heads) : vt_bytes;
     if (workspace && workspace_bytes < ws_bytes)
         return fail(CQKV_ERR_WORKSPACE, "cqkv_flash_attn: workspace %zu < %zu bytes",
                     workspace_bytes, ws_bytes);
+    // then the partials of split key ranges (not split in a workspace that does not hold them)
+    const size_t part_off = (ws_bytes + 255) / 256 * 256;
+    PfPlan plan = pf_plan(head_dim, batch, q_len, kv_len, q_heads, kv_heads, window_left, window_right);
+    if (plan.pieces > 1 && workspace && workspace_bytes < part_off + plan.bytes) plan = PfPlan{};
+    if (plan.pieces > 1) ws_bytes = part_off + plan.bytes;
+    a.piece_tiles = plan.tiles;
+    a.max_pieces = plan.pieces;
     const bool vt_owned = workspace == nullptr;
     if (vt_owned) CQKV_HIP_CHECK(hipMallocAsync(&vt, ws_bytes, st));
     a.vt = (const uint16_t *)vt;
+    if (plan.pieces > 1) {
+        const size_t rows = (size_t)plan.pieces * batch * q_heads * q_len;
+        a.part_o = (float *)((char *)vt + part_off);
+        a.part_lse = (float *)((char *)a.part_o + (rows * head_dim * 4 + 255) / 256 * 256);
+    }
     if (e4m3) {
         a.e4m3 = 1;
         a.f16 = dtype == CQKV_F16 ? 1 : 0;
@@ -1308,7 +1536,7 @@ int flash_attn_impl(const void *q, const int64_t q_strides[3], const void *k,
     if (head_dim == 64) hipLaunchKernelGGL(prefill_stage_kernel<64>, sgrid, dim3(256), 0, st, a);
     else if (head_dim == 256) hipLaunchKernelGGL(prefill_stage_kernel<256>, sgrid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL(prefill_stage_kernel<128>, sgrid, dim3(256), 0, st, a);
-    const dim3 grid(a.q_blocks * kv_heads * batch);
+    const dim3 grid(a.q_blocks * kv_heads * batch * a.max_pieces);
     const bool terms = softcap > 0.0f || alibi_slopes;
     if (head_dim == 64) pf_launch<64>(dtype == CQKV_F16, terms, grid, st, a);
     else if (head_dim == 256) pf_launch<256>(dtype == CQKV_F16, terms, grid, st, a);

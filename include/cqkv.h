@@ -356,7 +356,9 @@ int cqkv_flash_attn(const void *q, const int64_t q_strides[3], const void *k,
 
 /* Device workspace cqkv_flash_attn_ext needs for a call of these sizes (varlen != 0: per-sequence
  * lengths, q_len / kv_len their maxima; dtype is q's, the K / V dtype does not change it): the
- * MFMA prefill's V^T copy, or the plain kernel's split partials (0 when it does not split). */
+ * MFMA prefill's V^T copy, with the f32 partials of its split key ranges where few queries meet
+ * many keys (a workspace that holds only V^T serves the call unsplit), or the plain kernel's split
+ * partials (0 when it does not split). */
 size_t cqkv_flash_attn_workspace_bytes(int32_t dtype, int32_t batch, int32_t q_len,
                                        int32_t kv_len, int32_t q_heads, int32_t kv_heads,
                                        int32_t head_dim, int32_t varlen);

@@ -50,3 +50,30 @@ def test_wavefront_key_ranges(cq, dev, hq, hkv, sq, sk, wl, wr):
 def test_alibi_slope_per_column(cq, dev, hq, hkv):
     check(cq, dev, 1, 130, 200, hq, hkv, 128,
           alibi=[2.0 ** -(1 + i % 8) for i in range(hq)], dtype=torch.float16)
+
+
+@pytest.mark.parametrize("d,hq,hkv,sq,sk,wl,wr", [
+    (128, 8, 2, 40, 5000, -1, 0),    # few column blocks, long ranges: up to 16 pieces
+    (64, 2, 2, 300, 3001, -1, 0),    # several blocks, ragged last tile
+    (256, 4, 1, 33, 2100, -1, -1),
+    (128, 8, 8, 1100, 1100, -1, 0),  # causal: the early blocks have one piece, the late ones more
+    (128, 8, 2, 64, 4100, 1500, 0),  # a window: the range begins inside the keys
+    (128, 4, 1, 1000, 700, -1, 0),   # the first queries see no key
+])
+def test_split_key_ranges(cq, dev, d, hq, hkv, sq, sk, wl, wr):
+    check(cq, dev, 1, sq, sk, hq, hkv, d, wl, wr)
+
+
+def test_split_in_a_callers_workspace(cq, dev):
+    """The queried workspace gives the allocating call's bits; one that holds V^T but not the
+    partials still serves the call, unsplit, within the bar."""
+    q, k, v = (randn(i, s).to(dev) for i, s in
+               enumerate(((1, 64, 8, 128), (1, 4000, 2, 128), (1, 4000, 2, 128))))
+    want = cq.flash_attn(q, k, v, 0.09, True)
+    n = cq.flash_attn_workspace_bytes(torch.bfloat16, 1, 64, 4000, 8, 2, 128)
+    ws = torch.empty(n, dtype=torch.uint8, device=dev)
+    assert torch.equal(cq.flash_attn(q, k, v, 0.09, True, workspace=ws), want)
+    vt = 2 * 128 * 4032 * 2
+    assert n > vt
+    got = cq.flash_attn(q, k, v, 0.09, True, workspace=ws[:vt])
+    assert_close_bf16(got.float().cpu().numpy(), want.float().cpu().numpy())
