@@ -220,6 +220,7 @@ static int decode_prepare(DecodeArgs &a, DecodeHost &h, const char *who, const v
     a.q_heads = q_heads;
     a.kv_heads = hkv;
     a.group = group;
+    a.group_m = group > 1 && group <= 256 ? (uint32_t)(0x100000000ull / group + (0x100000000ull % group != 0)) : 0;
     a.q_len = q_len;
     a.ncols = group * q_len;
     a.col_blocks = (a.ncols + 15) / 16;

@@ -91,7 +91,14 @@ struct DecodeArgs {
     float kcent[8];        // compact key table (TURBOPROD, kFmtTurboC keys): their codebook
     float vcent[8];        // compact value table (kFmtTurboC values): their codebook
     int32_t kfmt, vfmt;    // host: the kernel formats of the call (kFmtTurboC where it applies)
+    uint32_t group_m;      // ceil(2^32 / group) for group 2 .. 256, else 0
 };
+
+// Query of column c (c / group; columns are below 2^24 + 16): one multiplication, exact as
+// c * (group_m * group - 2^32) < 2^32, instead of a division's dependent chain.
+__device__ inline int col_query(int c, const DecodeArgs &a) {
+    return a.group == 1 ? c : a.group_m ? (int)__umulhi((uint32_t)c, a.group_m) : c / a.group;
+}
 
 constexpr float kQjlConst = 1.2533141f;  // sqrt(pi / 2) as the reference's QJL_CONST (turbo.rs:26)
 
@@ -806,9 +813,11 @@ __attribute__((amdgpu_waves_per_eu(decode_min_waves<KF, VF, D>()))) void decode_
     // the per-wavefront outputs (and, before the tile loop, the queries) share their LDS with the
     // TurboQuant code table (64 KB-aligned, see turbo_pair), which is live only during the tile
     // loop
-    constexpr int kOWords = WAVES * 16 * D, kTabWords = kTurbo ? 256 * 64 : 0;
+    // (rows of D + 4 floats: with a row stride of a multiple of the banks, the 16 columns of one
+    // access met in the same banks)
+    constexpr int kRow = D + 4, kOWords = WAVES * 16 * kRow, kTabWords = kTurbo ? 256 * 64 : 0;
     __shared__ __attribute__((aligned(65536))) float sm_buf[kOWords > kTabWords ? kOWords : kTabWords];
-    float(*sm_o)[16][D] = (float(*)[16][D])sm_buf;
+    float(*sm_o)[16][kRow] = (float(*)[16][kRow])sm_buf;
     uint32_t *sm_tab = (uint32_t *)sm_buf;
     __shared__ float sm_m[WAVES][16], sm_l[WAVES][16];
     constexpr bool kProd = is_prod<KF>();
@@ -837,19 +846,20 @@ __attribute__((amdgpu_waves_per_eu(decode_min_waves<KF, VF, D>()))) void decode_
     // visible key range of this lane's column, and the workgroup-wide bounds
     const bool col_ok = n < ncb;
     int lo, hi, lo_min, hi_max, lo_max, hi_min;
-    key_range(col_ok ? (c0col + n) / a.group : 0, a.q_len, L, a.wl, a.wr, lo, hi);
+    key_range(col_ok ? col_query(c0col + n, a) : 0, a.q_len, L, a.wl, a.wr, lo, hi);
     // score terms of this lane's column: its ALiBi slope and its query's key position
     float slope2 = 0.0f;
     int qpos = 0;
     if constexpr (TERMS) {
         const int c = c0col + (col_ok ? n : 0);
-        qpos = c / a.group + L - a.q_len;
+        const int cq = col_query(c, a);
+        qpos = cq + L - a.q_len;
         if (a.alibi && col_ok)
-            slope2 = a.alibi[(int64_t)b * a.alibi_bs + hk * a.group + c % a.group] * kLog2e;
+            slope2 = a.alibi[(int64_t)b * a.alibi_bs + hk * a.group + (c - cq * a.group)] * kLog2e;
     }
     if (!col_ok) lo = hi = 0;
-    key_range(c0col / a.group, a.q_len, L, a.wl, a.wr, lo_min, hi_min);
-    key_range((c0col + ncb - 1) / a.group, a.q_len, L, a.wl, a.wr, lo_max, hi_max);
+    key_range(col_query(c0col, a), a.q_len, L, a.wl, a.wr, lo_min, hi_min);
+    key_range(col_query(c0col + ncb - 1, a), a.q_len, L, a.wl, a.wr, lo_max, hi_max);
     // the split's tiles and the planes they live in: a segment of one block (paged) or a range of
     // the cache's tiles
     const uint8_t *kc = a.kc, *ks = a.ks, *vc = a.vc, *vs = a.vs;
@@ -874,17 +884,56 @@ __attribute__((amdgpu_waves_per_eu(decode_min_waves<KF, VF, D>()))) void decode_
         te = min((split + 1) * a.tiles_per_split, (hi_max + 31) / 32);
     }
 
+    const int64_t plane = (int64_t)b * a.kv_heads + hk;
+    const rsrc_t kr = make_rsrc(kc + plane * kc_plane, kc_plane);
+    const rsrc_t ksr = make_rsrc(ks + plane * ks_plane, ks_plane);
+    const rsrc_t vr = make_rsrc(vc + plane * vc_plane, vc_plane);
+    const rsrc_t vsr = make_rsrc(vs + plane * vs_plane, vs_plane);
+    // NVFP4: the per-token f32 scales follow the block bytes of all the plane's tokens
+    uint32_t ktok_off = 0, vtok_off = 0;
+    if constexpr (KF == CQKV_FMT_NVFP4) ktok_off = ks_plane / (D / 16 + 4) * (D / 16);
+    if constexpr (kProd) ktok_off = ks_plane / (8 + D / 8);  // load_tile reads the capacity here
+    if constexpr (VF == CQKV_FMT_NVFP4) vtok_off = vs_plane / (D / 16 + 4) * (D / 16);
+
     // ---- queries (rotated keys: q Pi_k^T = sign-flip, Hadamard, 1/sqrt(D)) ----
-    float(*sm_q)[D] = sm_o[0];
-    for (int idx = threadIdx.x; idx < 16 * D; idx += NT) {
-        const int c = idx / D, d = idx % D;
-        float v = 0.0f;
-        if (c < ncb && d < a.head_dim) {
-            const int head = hk * a.group + (c0col + c) % a.group, qi = (c0col + c) / a.group;
-            v = load_elem(a.q, (int64_t)b * a.q_sb + (int64_t)head * a.q_sh + (int64_t)qi * a.q_si + d,
-                          a.q_dtype);
+    // thread i: element i % D of columns i / D + k * kCols; every load is issued (columns and
+    // elements past the end clamped) before the first conversion. The first two tiles of every
+    // wavefront are requested right behind them, so their latency passes behind the staging, the
+    // rotation and the code tables, which with the merge at the end are most of the time where a
+    // workgroup has few tiles (13 ragged sequences up to 3001 tokens, NVFP4: 22.0 -> 19.0 us for the
+    // kernel; 128K tokens of TurboQuant-4: 211.0 -> 205.8 us per call).
+    float(*sm_q)[kRow] = sm_o[0];
+    Tile<KF, VF, D> ta, tb2;
+    int t = tb + wave;
+    {
+        constexpr int kCols = NT / D, kIt = 16 / kCols;
+        const int d = threadIdx.x % D, c1 = threadIdx.x / D;
+        const int64_t q0 = (int64_t)b * a.q_sb + min(d, a.head_dim - 1);
+        uint32_t w[kIt];
+#pragma unroll
+        for (int k = 0; k < kIt; ++k) {
+            w[k] = 0;
+            if (kCols * k < ncb) {
+                const int c = c0col + min(c1 + kCols * k, ncb - 1), qi = col_query(c, a);
+                const int64_t at = q0 + (int64_t)(hk * a.group + (c - qi * a.group)) * a.q_sh +
+                                   (int64_t)qi * a.q_si;
+                if (a.q_dtype == CQKV_F32) w[k] = ((const uint32_t *)a.q)[at];
+                else w[k] = ((const uint16_t *)a.q)[at];
+            }
         }
-        sm_q[c][d] = v;
+        __builtin_amdgcn_sched_barrier(0);
+        load_tile<KF, VF, D>(ta, t, t < te, lane, kr, ksr, vr, vsr, ktok_off, vtok_off);
+        __builtin_amdgcn_sched_barrier(0);
+        load_tile<KF, VF, D>(tb2, t + WAVES, t + WAVES < te, lane, kr, ksr, vr, vsr, ktok_off, vtok_off);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < kIt; ++k) {
+            const int c = c1 + kCols * k;
+            float v = a.q_dtype == CQKV_F32   ? __uint_as_float(w[k])
+                      : a.q_dtype == CQKV_F16 ? f16_bits_to_f32(w[k])
+                                              : __uint_as_float(w[k] << 16);
+            sm_q[c][d] = c < ncb && d < a.head_dim ? v : 0.0f;
+        }
     }
     __syncthreads();
     if (a.rot_k) {
@@ -921,7 +970,7 @@ __attribute__((amdgpu_waves_per_eu(decode_min_waves<KF, VF, D>()))) void decode_
         // f16 queries: 2^-qe brings the largest |q| of the workgroup's columns below 2^15 (every
         // wavefront reads all of them, so each finds the same qe); exact scaling both ways
         float m = 0.0f;
-        for (int i = lane; i < 16 * D; i += 64) m = fmaxf(m, __builtin_fabsf(sm_q[i / D][i % D]));
+        for (int i = lane; i < ncb * D; i += 64) m = fmaxf(m, __builtin_fabsf(sm_q[i / D][i % D]));
         m = wave_max(m);
         qe = m < 16384.0f ? 0 : max(__builtin_amdgcn_frexp_expf(m) - 14, 0);  // m < 2^(qe + 14)
         kscale2 = __builtin_ldexpf(a.scale_log2, qe);
@@ -930,7 +979,7 @@ __attribute__((amdgpu_waves_per_eu(decode_min_waves<KF, VF, D>()))) void decode_
     for (int j = 0; j < NCH; ++j) {
         float qv[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) qv[e] = sm_q[n][qdim<KF, D>(j, g, e)];
+        for (int e = 0; e < 8; ++e) qv[e] = sm_q[n][qdim<KF, D>(j, g, 0) + e];
         if constexpr (KF == CQKV_FMT_NVFP4) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) qv[e] = __builtin_ldexpf(qv[e], -qe);
@@ -941,7 +990,7 @@ __attribute__((amdgpu_waves_per_eu(decode_min_waves<KF, VF, D>()))) void decode_
         // S q of the (rotated) queries on v_mfma_f32_16x16x4_f32: (S q)^T (D x 16) = S Q^T,
         // 16 outputs per wavefront step; k-step e of a group of four takes column
         // 16 kk + 4 g + e in lane group g (16-byte reads of S and of the queries)
-        float(*sm_qs)[D] = sm_o[1];
+        float(*sm_qs)[kRow] = sm_o[1];
         for (int bi = wave; bi < D / 16; bi += WAVES) {
             f32x4 acc2 = {0.f, 0.f, 0.f, 0.f};
             const float *srow = a.qjl + (int64_t)(16 * bi + n) * D + 4 * g;
@@ -975,24 +1024,20 @@ __attribute__((amdgpu_waves_per_eu(decode_min_waves<KF, VF, D>()))) void decode_
             sm_vtab[i] = pack_f16x2(a.vcent[(i >> 5) & 7], a.vcent[(i >> 9) & 7]);
     }
     __syncthreads();
-    if constexpr (kTurbo) {  // entry (b, l) at word 64 b + l: code pair (b & 15, b >> 4)
-        for (int i = threadIdx.x; i < 256 * 64; i += NT)
-            sm_tab[i] = pack_f16x2(a.cent[(i >> 6) & 15], a.cent[i >> 10]);
+    if constexpr (kTurbo) {
+        // entry (b, l) at word 64 b + l: code pair (b & 15, b >> 4); wavefront w writes bytes
+        // 256 / WAVES of them, so the centroids are scalars
+#pragma unroll
+        for (int hi = 0; hi < 16 / WAVES; ++hi) {
+            const float ch = a.cent[(16 / WAVES) * wave + hi];
+            uint32_t *row = sm_tab + ((16 / WAVES) * wave + hi) * 16 * 64 + lane;
+#pragma unroll
+            for (int lo4 = 0; lo4 < 16; ++lo4) row[64 * lo4] = pack_f16x2(a.cent[lo4], ch);
+        }
         __syncthreads();
     }
 
     // ---- stream the tiles of this split ----
-    const int64_t plane = (int64_t)b * a.kv_heads + hk;
-    const rsrc_t kr = make_rsrc(kc + plane * kc_plane, kc_plane);
-    const rsrc_t ksr = make_rsrc(ks + plane * ks_plane, ks_plane);
-    const rsrc_t vr = make_rsrc(vc + plane * vc_plane, vc_plane);
-    const rsrc_t vsr = make_rsrc(vs + plane * vs_plane, vs_plane);
-    // NVFP4: the per-token f32 scales follow the block bytes of all the plane's tokens
-    uint32_t ktok_off = 0, vtok_off = 0;
-    if constexpr (KF == CQKV_FMT_NVFP4) ktok_off = ks_plane / (D / 16 + 4) * (D / 16);
-    if constexpr (kProd) ktok_off = ks_plane / (8 + D / 8);  // load_tile reads the capacity here
-    if constexpr (VF == CQKV_FMT_NVFP4) vtok_off = vs_plane / (D / 16 + 4) * (D / 16);
-
     f32x4 acc[2 * NCH];
 #pragma unroll
     for (int t = 0; t < 2 * NCH; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1005,12 +1050,6 @@ __attribute__((amdgpu_waves_per_eu(decode_min_waves<KF, VF, D>()))) void decode_
 
     // Register sets A and B alternate; the scheduling barriers keep every load of one set
     // issued before the next set's, so each wait only covers the set about to be used.
-    Tile<KF, VF, D> ta, tb2;
-    int t = tb + wave;
-    load_tile<KF, VF, D>(ta, t, t < te, lane, kr, ksr, vr, vsr, ktok_off, vtok_off);
-    __builtin_amdgcn_sched_barrier(0);
-    load_tile<KF, VF, D>(tb2, t + WAVES, t + WAVES < te, lane, kr, ksr, vr, vsr, ktok_off, vtok_off);
-    __builtin_amdgcn_sched_barrier(0);
     for (; t < te; t += 2 * WAVES) {
         compute_tile<KF, VF, D, TERMS, QS>(ta, t, a, qhi, qlo, lane, lo, hi, lo_max, hi_min, Lb,
                                        koff, tab, m_run, l_run, acc, kProd ? qsop : qhi, ktab, vtab,
@@ -1036,12 +1075,14 @@ __attribute__((amdgpu_waves_per_eu(decode_min_waves<KF, VF, D>()))) void decode_
     }
     if constexpr (kTurbo) __syncthreads();  // every wavefront is done with the code table
     const float l_col = group16_sum(l_run);
+    if (n < ncb) {
 #pragma unroll
-    for (int u = 0; u < NCH; ++u)
+        for (int u = 0; u < NCH; ++u)
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sm_o[wave][n][32 * u + 8 * g + 2 * i + h] = acc[2 * u + h][i];
+            for (int i = 0; i < 4; i += 2)
+                *(f32x4 *)&sm_o[wave][n][32 * u + 8 * g + 2 * i] =
+                    f32x4{acc[2 * u][i], acc[2 * u + 1][i], acc[2 * u][i + 1], acc[2 * u + 1][i + 1]};
+    }
     if (g == 0) {
         sm_m[wave][n] = m_run;
         sm_l[wave][n] = l_col;
@@ -1068,7 +1109,7 @@ __attribute__((amdgpu_waves_per_eu(decode_min_waves<KF, VF, D>()))) void decode_
             o = osum / wsum;
             lse = M + __builtin_log2f(wsum);
         }
-        const int head = hk * a.group + (c0col + c) % a.group, qi = (c0col + c) / a.group;
+        const int qi = col_query(c0col + c, a), head = hk * a.group + (c0col + c - qi * a.group);
         if (d >= a.head_dim) continue;  // plane row padding
         if (!single) {  // the partial of this split; combine_kernel merges the splits
             const int64_t row = ((int64_t)b * a.q_heads + head) * a.q_len + qi;
