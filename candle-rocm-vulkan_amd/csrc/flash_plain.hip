@@ -157,6 +157,11 @@ int fa_plain_run(FaArgs a, const char *who, void *workspace, size_t workspace_by
         a.q_vec = fa_vec_ok(a.q, qs, f32 ? 4 : 2) ? 1 : 0;
         a.o_vec = f32 && fa_vec_ok(a.out, os, 4) ? 1 : 0;
     }
+    if (f32) {
+        bool taken;
+        const int rc = prefill_f32_run(a, who, workspace, workspace_bytes, st, &taken);
+        if (rc != CQKV_OK || taken) return rc;
+    }
     void *ws = workspace;
     bool owned = false;
     if (s > 1) {

@@ -31,11 +31,11 @@
 //  * Causal work is uneven: the workgroups with the most key tiles are dispatched first.
 #include <algorithm>
 #include <type_traits>
-#include <vector>
 
 #include "cqkv_device.h"
 #include "cqkv_host.h"
 #include "flash_plain.h"
+#include "prefill_split.h"
 
 namespace cqkv {
 
@@ -90,14 +90,10 @@ struct PrefillArgs {
     // D) prefill_combine_kernel merges; column blocks of one piece write the output themselves
     int32_t piece_tiles, max_pieces;
     float *part_o, *part_lse;
-    uint32_t group_m;  // ceil(2^32 / group) for group 2 .. 32768, else 0
+    uint32_t group_m;  // pf_group_m(group)
 };
 
-// c / group for the columns of a workgroup (c < group + 256): one multiplication instead of a
-// division's dependent chain in the prologue (exact, as c * (group_m * group - 2^32) < 2^32).
-__device__ inline int pf_query_of(int c, const PrefillArgs &a) {
-    return a.group == 1 ? c : a.group_m ? (int)__umulhi((uint32_t)c, a.group_m) : c / a.group;
-}
+__device__ inline int pf_query_of(int c, const PrefillArgs &a) { return pf_div_group(c, a.group, a.group_m); }
 
 // First rows and lengths of sequence b. Variable-length offsets are clamped into the tensors
 // and the lengths to q_len / kv_len, so inconsistent prefix sums cannot address memory outside
@@ -140,31 +136,6 @@ template <bool F16>
 using pf_op_t = typename std::conditional<F16, f16x8, bf16x8>::type;
 
 __device__ inline u32x4 ldg128(const uint16_t *p) { return *(const u32x4 *)p; }
-
-// visible keys [lo, hi) of query position i (bottom-right aligned)
-__host__ __device__ inline void pf_key_range(int i, int lq, int lk, int wl, int wr, int &lo, int &hi) {
-    const int pos = i + lk - lq;
-    lo = wl >= 0 ? max(pos - wl, 0) : 0;
-    hi = wr >= 0 ? min(pos + wr + 1, lk) : lk;
-    lo = min(lo, lk);
-    hi = max(hi, lo);
-}
-
-// Pieces that n key tiles are cut into: whole pieces of piece_tiles and a last one of up to a
-// quarter more (the rest up to a quarter is not worth a workgroup and its partials).
-__host__ __device__ inline int pf_pieces(int n, int piece_tiles, int max_pieces) {
-    const int rest = n - piece_tiles / 4;
-    return max_pieces <= 1 || rest <= piece_tiles ? 1 : min((rest + piece_tiles - 1) / piece_tiles, max_pieces);
-}
-// Key tiles (of bk keys) of the column block whose queries are q0 .. q1: first tile and count.
-__host__ __device__ inline int pf_block_tiles(int q0, int q1, int lq, int lk, int wl, int wr, int bk,
-                                              int &begin) {
-    int lo, hi, lo1;
-    pf_key_range(q0, lq, lk, wl, wr, lo, hi);
-    pf_key_range(q1, lq, lk, wl, wr, lo1, hi);
-    begin = lo / bk;
-    return max((hi + bk - 1) / bk - begin, 0);
-}
 
 // LDS K tile layout: 64 rows (keys) x 2 D bytes, no padding; the 16-byte chunk c of row r sits at
 // chunk position c ^ swz(r). At D = 128 (16 chunks a row) swz takes 16 distinct values over any 16
@@ -901,7 +872,6 @@ __global__ __launch_bounds__(PfGeom<D>::W * 64, 1) void prefill_kernel(PrefillAr
 // w_p = 2^(lse_p - max lse) (tq_combine_impl's formula, candle-core/kernels/turbo_quant_impl.h:
 // 659-685), pieces without a visible key skipped. D / 4 lanes per column, 4 head dims each; lane p of
 // each 16 loads piece p's lse (at most kPfMaxPieces = 16), so the weights cost one load's latency.
-constexpr int kPfMaxPieces = 16;
 template <bool F16, int D>
 __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a) {
     using G = PfGeom<D>;
@@ -1156,82 +1126,17 @@ static size_t pf_kst_bytes(int32_t batch, int32_t kv_len, int32_t kv_heads) {
     return (size_t)batch * kv_heads * kv_len * kPfD * 2;
 }
 
-// How a call's key ranges are split: column blocks of more than `tiles` key tiles in up to `pieces`
-// pieces (1: not at all), and the bytes of the partials.
-struct PfPlan {
-    int tiles = 1 << 30, pieces = 1;
-    size_t bytes = 0;
-};
-// A CU holds one workgroup, so a call of few column blocks leaves CUs idle: one 300-token chunk of a
-// 32 / 8-head model over 7000 keys is 40 blocks of 110 tiles on 256 CUs (157 -> 54 us per call in 6
-// pieces). The count with the smallest estimate is taken:
-//  * steps: key tiles that the last CU to end works through, a workgroup costing kSetup tiles beside
-//    its own (its queries, the first tiles' latency, the output). Up to 256 workgroups: the longest;
-//    more: the mean per CU and half a workgroup.
-//  * a step takes lo us on an idle chip and up to hi us more the fuller it is (clocks, caches: at
-//    D = 128, 1.3 us with 40 workgroups, 1.86 us with 200), so t = lo * steps + hi * mean tiles per CU.
-//  * the combine: 3 us, and its partials written and read, mostly cached, at 8 TB/s (6.8 us for 9600
-//    rows of 5 pieces).
-// A causal prompt of about as many blocks as CUs keeps them whole: its mean is half of its longest,
-// but the rate rises as CUs fall idle, and the partials cost what is left (2048 tokens, 32 / 8 heads:
-// 62.6 us whole, 66.2 us in halves; 3000 tokens: 91.7 and 110.2). No piece is under 512 keys, so
-// shorter sequences are never split.
-static PfPlan pf_plan(int head_dim, int batch, int q_len, int kv_len, int q_heads, int kv_heads,
-                      int wl, int wr) {
-    constexpr int kCus = 256, kSetup = 3;
-    const int nc = head_dim == 256 ? PfGeom<256>::NC : PfGeom<128>::NC;
-    const int bk = head_dim == 256 ? PfGeom<256>::BK : PfGeom<128>::BK;
-    const int min_tiles = 512 / bk, group = q_heads / kv_heads;
-    const double lo = head_dim == 64 ? 0.76 : head_dim == 128 ? 1.2 : 0.7;
-    const double hi = head_dim == 64 ? 0.4 : head_dim == 128 ? 0.75 : 0.4;
-    const int64_t planes = (int64_t)batch * kv_heads, cols = (int64_t)q_len * group;
-    const int64_t blocks = (cols + nc - 1) / nc;
-    PfPlan best;
-    if (planes * blocks > 2 * kCus || kv_len <= 512) return best;
-    std::vector<int> n(blocks);  // key tiles, in the order the blocks are handed out
-    int most = 0;
-    for (int64_t i = 0; i < blocks; ++i) {
-        const int64_t c0 = (blocks - 1 - i) * nc;
-        int begin;
-        n[i] = pf_block_tiles((int)(c0 / group), (int)((std::min(c0 + nc, cols) - 1) / group), q_len,
-                              kv_len, wl, wr, bk, begin);
-        most = std::max(most, n[i]);
-    }
-    double best_us = 0.0;
-    for (int p = 1; p <= kPfMaxPieces; ++p) {
-        const int tiles = (most + p - 1) / p;
-        if (p > 1 && (tiles < min_tiles || planes * blocks * p > 8 * kCus)) break;
-        int64_t wgs = 0, total = 0, split_cols = 0;
-        int longest = 0;
-        for (int64_t i = 0; i < blocks; ++i) {
-            const int k = pf_pieces(n[i], tiles, p);
-            const int last = n[i] - (k - 1) * tiles;
-            longest = std::max(longest, k > 1 ? std::max(last, tiles) : last);
-            wgs += planes * k;
-            total += planes * (n[i] + (int64_t)k * kSetup);
-            if (k > 1) split_cols += k * nc;
-        }
-        const double mean = (double)total / kCus;
-        double steps = longest + kSetup;
-        if (wgs > kCus) steps = std::max(steps, mean + 0.5 * total / wgs);
-        double t = lo * steps + hi * mean;
-        if (p > 1) t += 3.0 + (double)planes * split_cols * head_dim * 8 / 8e6;
-        if (p == 1 || t < (best.pieces == 1 ? 0.92 : 0.97) * best_us) {
-            best_us = t;
-            best.tiles = tiles;
-            best.pieces = p;
-        }
-    }
-    if (best.pieces > 1)
-        best.bytes = ((size_t)best.pieces * planes * cols * head_dim * 4 + 255) / 256 * 256 +
-                     (size_t)best.pieces * planes * cols * 4;
-    return best;
+// The column blocks and step times of the MFMA prefill at a head dim.
+static PfShape pf_shape(int head_dim) {
+    if (head_dim == 64) return {PfGeom<64>::NC, PfGeom<64>::BK, 64, 0.76, 0.4, 3, 512, false};
+    if (head_dim == 128) return {PfGeom<128>::NC, PfGeom<128>::BK, 128, 1.2, 0.75, 3, 512, false};
+    return {PfGeom<256>::NC, PfGeom<256>::BK, 256, 0.7, 0.4, 3, 512, false};
 }
 // Bytes of the partials whatever the window: the larger of the causal and the full mask's plan (a
 // call whose own plan needs more than its workspace holds is not split).
 static size_t pf_part_bytes(int head_dim, int batch, int q_len, int kv_len, int q_heads, int kv_heads) {
-    return std::max(pf_plan(head_dim, batch, q_len, kv_len, q_heads, kv_heads, -1, 0).bytes,
-                    pf_plan(head_dim, batch, q_len, kv_len, q_heads, kv_heads, -1, -1).bytes);
+    return std::max(pf_plan(pf_shape(head_dim), batch, q_len, kv_len, q_heads, kv_heads, -1, 0).bytes,
+                    pf_plan(pf_shape(head_dim), batch, q_len, kv_len, q_heads, kv_heads, -1, -1).bytes);
 }
 
 bool prefill_takes(int32_t dtype, int32_t head_dim, int32_t q_len, const void *q,
@@ -1264,6 +1169,8 @@ size_t flash_attn_workspace(int32_t dtype, int32_t batch, int32_t q_len, int32_t
         return std::max((pf_vt_bytes(batch, kv_len, kv_heads, head_dim) + 255) / 256 * 256 +
                             pf_part_bytes(head_dim, batch, q_len, kv_len, q_heads, kv_heads),
                         plain);
+    if (dtype == CQKV_F32)
+        return std::max(plain, prefill_f32_workspace(batch, q_len, kv_len, q_heads, kv_heads, head_dim));
     return plain;
 }
 
@@ -1452,7 +1359,7 @@ int flash_attn_impl(const void *q, const int64_t q_strides[3], const void *k,
     a.q_heads = q_heads;
     a.kv_heads = kv_heads;
     a.group = q_heads / kv_heads;
-    a.group_m = a.group > 1 && a.group <= 32768 ? (uint32_t)(0x100000000ull / a.group + (0x100000000ull % a.group != 0)) : 0;
+    a.group_m = pf_group_m(a.group);
     const int nc = head_dim == 256 ? PfGeom<256>::NC : PfGeom<128>::NC;  // columns per workgroup
     a.q_blocks = (int)(((int64_t)q_len * a.group + nc - 1) / nc);
     a.wl = window_left;
@@ -1482,7 +1389,7 @@ int flash_attn_impl(const void *q, const int64_t q_strides[3], const void *k,
                     workspace_bytes, ws_bytes);
     // then the partials of split key ranges (not split in a workspace that does not hold them)
     const size_t part_off = (ws_bytes + 255) / 256 * 256;
-    PfPlan plan = pf_plan(head_dim, batch, q_len, kv_len, q_heads, kv_heads, window_left, window_right);
+    PfPlan plan = pf_plan(pf_shape(head_dim), batch, q_len, kv_len, q_heads, kv_heads, window_left, window_right);
     if (plan.pieces > 1 && workspace && workspace_bytes < part_off + plan.bytes) plan = PfPlan{};
     if (plan.pieces > 1) ws_bytes = part_off + plan.bytes;
     a.piece_tiles = plan.tiles;

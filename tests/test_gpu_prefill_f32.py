@@ -1,0 +1,114 @@
+"""f32 queries on split bf16 operands (prefill_f32.hip): column and key remainders, the split of key
+ranges, both workgroup widths, masks, score terms, head dims below the padded ones, variable lengths
+and every K / V type, against float64 within the reference's f32 bar of 1e-5 of max |ref|; infinities;
+and the route of a call whose workspace or alignment does not serve the path."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def randn(seed, shape, dtype=torch.float32):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(dtype)
+
+
+def attention_f64(q, k, v, scale, causal, wl=-1, softcap=0.0, alibi=None):
+    b, sq, hq, d = q.shape
+    sk, hkv = k.shape[1], k.shape[2]
+    q, k, v = (x.double().transpose(1, 2) for x in (q, k, v))
+    k, v = (x.repeat_interleave(hq // hkv, 1) for x in (k, v))
+    s = q @ k.transpose(2, 3) * scale
+    if softcap:
+        s = softcap * torch.tanh(s / softcap)
+    dist = torch.arange(sq)[:, None] + (sk - sq) - torch.arange(sk)[None]
+    if alibi is not None:
+        s -= alibi.double()[None, :, None, None] * dist.abs()
+    hide = (dist < 0) & causal
+    if wl >= 0:
+        hide |= dist > wl
+    s = s.masked_fill(hide, -math.inf)
+    return torch.nan_to_num(s.softmax(-1)).matmul(v).transpose(1, 2)
+
+
+def check(cq, dev, b, sq, sk, hq, hkv, d, kvd=torch.float32, causal=True, wl=-1, softcap=0.0,
+          alibi=None, scale=1.0):
+    q = randn(1, (b, sq, hq, d)) * scale
+    k, v = randn(2, (b, sk, hkv, d), kvd), randn(3, (b, sk, hkv, d), kvd)
+    got = cq.flash_attn(q.to(dev), k.to(dev), v.to(dev), 1 / math.sqrt(d), causal, window_left=wl,
+                        softcap=softcap, alibi_slopes=None if alibi is None else alibi.to(dev))
+    want = attention_f64(q, k, v, 1 / math.sqrt(d), causal, wl, softcap, alibi)
+    assert (got.cpu().double() - want).abs().max() <= 1e-5 * want.abs().max()
+
+
+@pytest.mark.parametrize("d", [8, 64, 72, 128])
+@pytest.mark.parametrize("hq,hkv", [(2, 2), (6, 2), (16, 1)])
+@pytest.mark.parametrize("sq,sk", [(129, 129), (86, 97), (257, 300), (65, 1000)])
+def test_column_and_key_remainders(cq, dev, d, hq, hkv, sq, sk):
+    check(cq, dev, 1, sq, sk, hq, hkv, d)
+
+
+@pytest.mark.parametrize("kvd", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("b,sq,sk,hq,hkv,d,causal,wl", [
+    (1, 40, 5000, 8, 2, 128, True, -1),     # one block, up to 16 pieces
+    (1, 700, 2100, 4, 4, 64, True, -1),     # pieces by falling size
+    (2, 400, 1500, 8, 2, 128, True, 600),   # a window
+    (1, 300, 200, 4, 2, 128, True, -1),     # queries that see no key
+    (1, 200, 1111, 4, 2, 64, False, -1),
+    (8, 600, 600, 16, 16, 64, True, -1),    # more than two blocks per CU: 8 wavefronts, unsplit
+])
+def test_splits_and_masks(cq, dev, kvd, b, sq, sk, hq, hkv, d, causal, wl):
+    check(cq, dev, b, sq, sk, hq, hkv, d, kvd, causal, wl)
+
+
+def test_score_terms_and_large_scores(cq, dev):
+    slopes = 0.05 * (1 + torch.arange(6, dtype=torch.float32))
+    check(cq, dev, 1, 150, 400, 6, 2, 64, softcap=3.0, alibi=slopes)
+    check(cq, dev, 1, 150, 400, 6, 2, 128, scale=20.0)
+
+
+def test_variable_lengths_equal_f64(cq, dev):
+    lens = [200, 0, 1, 333, 64]
+    cu = torch.tensor([0, *torch.tensor(lens).cumsum(0)], dtype=torch.int32, device=dev)
+    n, hq, hkv, d = sum(lens), 8, 2, 64
+    q, k, v = randn(1, (n, hq, d)), randn(2, (n, hkv, d)), randn(3, (n, hkv, d))
+    got = cq.flash_attn_varlen(q.to(dev), k.to(dev), v.to(dev), cu, cu, 333, 333, 0.125, True).cpu()
+    at = 0
+    for m in lens:
+        if m:
+            want = attention_f64(q[None, at:at + m], k[None, at:at + m], v[None, at:at + m], 0.125, True)
+            assert (got[at:at + m].double() - want[0]).abs().max() <= 1e-5 * want.abs().max()
+        at += m
+
+
+def test_non_finite_inputs(cq, dev):
+    """A key at -inf * sign(q) gives probability 0, an infinite value an infinite output; queries near
+    the top of f32 keep their scores (no part overflows: their bf16 rounding would)."""
+    q = randn(1, (1, 130, 2, 64)).abs() + 0.5
+    k, v = randn(2, (1, 200, 2, 64)), randn(3, (1, 200, 2, 64))
+    k[0, 5] = -math.inf
+    v[0, 9, 0, 3] = math.inf
+    q[0, 100, 1, 5], k[0, :, 1, 5] = 3.4e38, k[0, :, 1, 5] * 2.0 ** -100
+    got = cq.flash_attn(q.to(dev), k.to(dev), v.to(dev), 0.1, False).cpu()
+    keep = torch.arange(200) != 5
+    want = attention_f64(q, k[:, keep], v[:, keep], 0.1, False)
+    assert torch.isposinf(got[0, :, 0, 3]).all()
+    fin = torch.isfinite(want)
+    assert (got.double() - want)[fin].abs().max() <= 1e-5 * want[fin].abs().max()
+
+
+def test_workspaces_and_unaligned_rows(cq, dev):
+    q, k, v = (randn(i, s).to(dev) for i, s in
+               enumerate(((1, 200, 4, 64), (1, 900, 2, 64), (1, 900, 2, 64))))
+    want = cq.flash_attn(q, k, v, 0.125, True)
+    n = cq.flash_attn_workspace_bytes(torch.float32, 1, 200, 900, 4, 2, 64)
+    ws = torch.empty(n, dtype=torch.uint8, device=dev)
+    assert torch.equal(cq.flash_attn(q, k, v, 0.125, True, workspace=ws), want)
+    images = 2 * 29 * 6 * 2 * 32 * 64
+    assert n > images
+    odd = torch.empty(1, 200, 4, 66, device=dev)[..., :64]
+    odd.copy_(q)
+    for got in (cq.flash_attn(q, k, v, 0.125, True, workspace=ws[:images]),
+                cq.flash_attn(odd, k, v, 0.125, True)):
+        assert (got - want).abs().max() <= 1e-5 * want.abs().max()
