@@ -112,6 +112,7 @@ def lib() -> ctypes.CDLL:
         L.cqkv_flash_attn_blocks.argtypes = [P, I64P, PBP, i32, i32, i32, i32, i32, i32, i32,
                                              i32, f32, i32, i32, f32, P, i32, P, I64P, P, sz, P]
         L.cqkv_fp8_quantize_tensor.argtypes = [P, i32, ctypes.c_int64, P, P, P]
+        L.cqkv_fp8_quantize_pair.argtypes = [P, P, i32, ctypes.c_int64, ctypes.c_int64, P, P, P, P, P]
         L.cqkv_hadamard_rows.argtypes = [P, i32, ctypes.c_int64, ctypes.c_int64, i32,
                                          ctypes.c_uint64, P, ctypes.c_int64, P]
         L.cqkv_flash_attn_fp8.argtypes = [P, I64P, P, I64P, P, I64P, P, I64P, i32, i32, i32, i32,
@@ -145,7 +146,7 @@ EXPORTED = ["cqkv_codes_plane_bytes", "cqkv_scales_plane_bytes", "cqkv_quant_app
             "cqkv_decode_paged_workspace_bytes", "cqkv_decode_attention_paged",
             "cqkv_flash_attn", "cqkv_flash_attn_ext", "cqkv_flash_attn_workspace_bytes",
             "cqkv_flash_attn_blocks", "cqkv_flash_attn_blocks_workspace_bytes",
-            "cqkv_fp8_quantize_tensor",
+            "cqkv_fp8_quantize_tensor", "cqkv_fp8_quantize_pair",
             "cqkv_flash_attn_fp8", "cqkv_flash_attn_fp8_workspace_bytes", "cqkv_hadamard_rows", "cqkv_reference_row_words", "cqkv_rows_import",
             "cqkv_rows_export", "cqkv_side_copy", "cqkv_turbo_codebook", "cqkv_turbo_signs",
             "cqkv_qjl_matrix", "cqkv_rotation_matrix", "cqkv_resolve_rotation",
@@ -602,6 +603,22 @@ def fp8_quantize_tensor(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     return codes, scale
 
 
+def _fp8_quantize_pair(k: torch.Tensor, v: torch.Tensor):
+    """fp8_quantize_tensor of k and of v, in one set of launches where they share a dtype."""
+    if k.dtype != v.dtype or k.device != v.device or k.device.type != "cuda":
+        (k8, ks), (v8, vs) = fp8_quantize_tensor(k), fp8_quantize_tensor(v)
+        return k8, v8, ks, vs
+    if k.dtype not in _DTYPES:
+        raise CqkvError(ERR_ARG, "k / v must be bf16 / f16 / f32 tensors")
+    k8, v8 = (torch.empty(t.shape, dtype=torch.uint8, device=t.device) for t in (k, v))
+    scales = torch.empty((2, 2), dtype=torch.float32, device=k.device)
+    ks, vs = scales[0], scales[1]
+    _check(lib().cqkv_fp8_quantize_pair(_ptr(k), _ptr(v), _DTYPES[k.dtype], k.numel(), v.numel(),
+                                        _ptr(k8), _ptr(v8), _ptr(ks), _ptr(vs),
+                                        _stream(k.device)))
+    return k8, v8, ks, vs
+
+
 def _fp8_codes(t: torch.Tensor, name: str) -> torch.Tensor:
     if getattr(torch, "float8_e4m3fn", None) is not None and t.dtype == torch.float8_e4m3fn:
         return t.view(torch.uint8)
@@ -675,8 +692,7 @@ def flash_attn_fp8(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, softmax_sc
     d = q.shape[-1]
     if hadamard and d > 1 and d & (d - 1) == 0:  # power-of-two head dims, as the reference
         q, k = hadamard_rows(q), hadamard_rows(k)
-    k8, ks = fp8_quantize_tensor(k.contiguous())
-    v8, vs = fp8_quantize_tensor(v.contiguous())
+    k8, v8, ks, vs = _fp8_quantize_pair(k.contiguous(), v.contiguous())
     return flash_attn_fp8_codes(q, k8, v8, softmax_scale, causal, 1.0, 1.0, window_left,
                                 window_right, ks, vs, out)
 

@@ -430,6 +430,12 @@ int cqkv_flash_attn_blocks(const void *q, const int64_t q_strides[3],
 int cqkv_fp8_quantize_tensor(const void *x, int32_t x_dtype, int64_t n, uint8_t *codes,
                              float *scale, cqkv_stream_t stream);
 
+/* The same for K and V (k_n and v_n elements of one dtype) in the launches of one tensor; k_scale and
+ * v_scale: device float[2] each. */
+int cqkv_fp8_quantize_pair(const void *k, const void *v, int32_t dtype, int64_t k_n, int64_t v_n,
+                           uint8_t *k_codes, uint8_t *v_codes, float *k_scale, float *v_scale,
+                           cqkv_stream_t stream);
+
 /* Attention over E4M3 K / V with descale factors (flash_attn_with_config on F8E4M3 tensors):
  * shapes, strides, head dims and masks as cqkv_flash_attn (q, out of `dtype`, bf16, f16 or f32;
  * k8 / v8 E4M3 bytes, strides multiples of 8, 8-byte aligned). Keys are e4m3(k8) * k_descale *
