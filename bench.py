@@ -45,7 +45,6 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
 BF16_PEAK_TFLOPS = 2516.6
-F32_PEAK_TFLOPS = 157.3  # dense f32 MFMA
 TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "decode_fp8_c2_and_append_rows_traffic.md")
 
 
@@ -400,7 +399,7 @@ def plain_decode_case(cq, dev, stream, steps, warmup, dtype, B=32, HQ=32, HKV=8,
 def plain_prefill_case(cq, dev, stream, steps, warmup, dtype, D, B=4, S=4096, HQ=32, HKV=8,
                        q_dtype=None):
     """Causal flash_attn on the plain-dtype kernel (f16, or a head dim other than 128), or with
-    f32 queries on the f32 kernel (roofline: the f32 MFMA peak)."""
+    f32 queries on split bf16 operands (roofline: the bf16 MFMA peak over its six products)."""
     import torch
     q_dtype = q_dtype or dtype
     q = kv_gpu((B, S, HQ, D), 71, dev, outliers=False).to(q_dtype)
@@ -416,8 +415,9 @@ def plain_prefill_case(cq, dev, stream, steps, warmup, dtype, D, B=4, S=4096, HQ
     torch.cuda.empty_cache()
     tf = flops / (ms * 1e-3) / 1e12
     f32 = q_dtype == torch.float32
-    peak = F32_PEAK_TFLOPS if f32 else BF16_PEAK_TFLOPS
-    kind = "f32 kernel, f32 MFMA" if f32 else "plain-dtype kernel"
+    # f32 queries: six bf16 products each (three exact bf16 parts per operand)
+    peak = BF16_PEAK_TFLOPS / 6 if f32 else BF16_PEAK_TFLOPS
+    kind = "f32 on split bf16 operands" if f32 else "plain-dtype kernel"
     qn = "" if q_dtype == dtype else f"{str(q_dtype)[6:]} queries over "
     return {"workload": f"causal flash_attn, {qn}{str(dtype)[6:]}, D={D}, B={B} S={S} "
                         f"{HQ}/{HKV} heads ({kind})",

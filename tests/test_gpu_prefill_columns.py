@@ -77,3 +77,46 @@ def test_split_in_a_callers_workspace(cq, dev):
     assert n > vt
     got = cq.flash_attn(q, k, v, 0.09, True, workspace=ws[:vt])
     assert_close_bf16(got.float().cpu().numpy(), want.float().cpu().numpy())
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_split_with_score_terms(cq, dev, d):
+    check(cq, dev, 1, 40, 3000, 6, 2, d, alibi=[2.0 ** -(4 + i) for i in range(6)])
+
+
+def test_split_variable_lengths(cq, dev):
+    """Few queries against long key ranges of different lengths (more key tiles per block than the
+    longest query and key lengths together suggest), an empty sequence and one without keys."""
+    lens_q, lens_k, hq, hkv, d = [40, 0, 130, 70], [3000, 60, 700, 0], 8, 2, 128
+    q, k, v = randn(1, (sum(lens_q), hq, d)), randn(2, (sum(lens_k), hkv, d)), randn(3, (sum(lens_k), hkv, d))
+    cu = [torch.tensor([0, *np.cumsum(n)], dtype=torch.int32, device=dev) for n in (lens_q, lens_k)]
+    got = cq.flash_attn_varlen(q.to(dev), k.to(dev), v.to(dev), *cu, max(lens_q), max(lens_k), 0.09,
+                               True).float().cpu().numpy()
+    iq = ik = 0
+    for nq, nk in zip(lens_q, lens_k):
+        if nq:
+            qf, kf, vf = (x.float().permute(1, 0, 2)[None].contiguous().numpy() for x in
+                          (q[iq:iq + nq], k[ik:ik + nk], v[ik:ik + nk]))
+            want = (O.round_bf16(O.attention_unfused(qf, kf, vf, 0.09, wl=-1, wr=0, threads=16))[0]
+                    .transpose(1, 0, 2) if nk else np.zeros((nq, hq, d), np.float32))
+            assert_close_bf16(got[iq:iq + nq], want)
+        iq, ik = iq + nq, ik + nk
+
+
+def test_split_with_e4m3_keys_and_cache_append(cq, dev):
+    """Split calls whose workspace also holds the widened E4M3 K, and whose pre-pass appends."""
+    b, sq, sk, hq, hkv, d = 1, 40, 3000, 8, 2, 128
+    q, k, v = randn(1, (b, sq, hq, d)), randn(2, (b, sk, hkv, d)), randn(3, (b, sk, hkv, d))
+    k8, v8 = (x.to(dev).to(torch.float8_e4m3fn) for x in (k, v))
+    got = cq.flash_attn_fp8_codes(q.to(dev), k8, v8, 0.09, True)
+    want = cq.flash_attn(q.to(dev), k8.to(torch.bfloat16), v8.to(torch.bfloat16), 0.09, True)
+    assert_close_bf16(got.float().cpu().numpy(), want.float().cpu().numpy())
+    sides = [cq.CacheSide.empty(cq.FP8, bool(i & 1), b, hkv, d, sk, dev) for i in range(4)]
+    plain = cq.flash_attn(q.to(dev), k.to(dev), v.to(dev), 0.09, True)
+    fused = cq.flash_attn(q.to(dev), k.to(dev), v.to(dev), 0.09, True, k_cache=sides[0],
+                          v_cache=sides[1])
+    assert torch.equal(fused, plain)
+    for side, x in ((sides[2], k), (sides[3], v)):
+        cq.quant_append(side, x.to(dev).transpose(1, 2), 0)
+    for a, r in zip(sides[:2], sides[2:]):
+        assert torch.equal(a.codes, r.codes) and torch.equal(a.scales, r.scales)
