@@ -571,15 +571,17 @@ static size_t x3_images(const FaArgs &a) {
     return (size_t)a.batch * a.kv_heads * ((a.kv_len + kX3Bk - 1) / kX3Bk) * image;
 }
 
-// Whether a call's sizes take this path. Up to 64 columns per plane (one block of fa32_kernel), and up
-// to 127 where the planes alone fill the chip, the images' traffic costs more than the products gain
-// (66 columns, 32 planes, 1000 keys: 44 us here, 38 us there; 68 columns, 8 planes, 2000 keys: 39 and
-// 42); below 96 keys a launch more. The images are held to 2 GiB.
+// Whether a call's sizes take this path. Up to 64 columns per plane (one block of fa32_kernel), and
+// with more than 16 planes, which fill the chip by themselves, up to 127 (255 at D = 128), the images'
+// traffic and the blocks' padding cost more than the products gain (66 columns, 32 planes, 1000 keys,
+// D = 128: 44 us here, 38 us there; 142 columns, 48 planes, 653 keys: 71 and 63; 312 columns, 24
+// planes, 2780 keys: 155 and 153; 68 columns, 8 planes, 2000 keys: 39 and 42); below 96 keys a launch
+// more. The images are held to 2 GiB.
 static bool x3_sizes(const FaArgs &a) {
+    const int64_t cols = (int64_t)a.q_len * a.group, planes = (int64_t)a.batch * a.kv_heads;
+    const int64_t most = planes <= 16 ? 64 : a.head_dim <= 64 ? 127 : 255;  // columns left to fa32_kernel
     return a.dtype == CQKV_F32 && a.head_dim <= 128 && a.head_dim % 8 == 0 && a.kv_len >= 96 &&
-           (int64_t)a.q_len * a.group > ((int64_t)a.batch * a.kv_heads <= 16 ? 64 : 127) &&
-           (int64_t)a.batch * a.kv_heads <= 65535 &&
-           x3_images(a) <= ((size_t)2 << 30);
+           cols > most && planes <= 65535 && x3_images(a) <= ((size_t)2 << 30);
 }
 
 size_t prefill_f32_workspace(int32_t batch, int32_t q_len, int32_t kv_len, int32_t q_heads,
