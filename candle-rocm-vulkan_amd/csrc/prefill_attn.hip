@@ -835,10 +835,10 @@ __global__ __launch_bounds__(PfGeom<D>::W * 64, 1) void prefill_kernel(PrefillAr
     const float inv = l > 0.0f ? om / l : 0.0f;
     if (32 * wave + qr >= ncol) return;
     if (SPLIT && pieces > 1) {  // this piece's normalised rows and their log2-sum-exp, f32
-        const float invl = l > 0.0f ? 1.0f / l : 0.0f;
+        const float invl = l == 0.0f ? 0.0f : 1.0f / l;
         const int64_t row = ((int64_t)piece * nplanes + plane) * ((int64_t)a.q_len * a.group) +
                             (c0 + 32 * wave + qr);
-        if (h == 0) a.part_lse[row] = l > 0.0f ? st.m_run + __builtin_amdgcn_logf(l) : -__builtin_inff();
+        if (h == 0) a.part_lse[row] = pf_piece_lse(st.m_run, l);
         float *po = a.part_o + row * D + 4 * h;
 #pragma unroll
         for (int md = 0; md < G::MD; ++md)
@@ -868,15 +868,12 @@ __global__ __launch_bounds__(PfGeom<D>::W * 64, 1) void prefill_kernel(PrefillAr
         }
 }
 
-// Merges the pieces of the column blocks that have more than one: o = sum_p w_p o_p / sum_p w_p with
-// w_p = 2^(lse_p - max lse) (tq_combine_impl's formula, candle-core/kernels/turbo_quant_impl.h:
-// 659-685), pieces without a visible key skipped. D / 4 lanes per column, 4 head dims each; lane p of
-// each 16 loads piece p's lse (at most kPfMaxPieces = 16), so the weights cost one load's latency.
+// Merges the pieces of the column blocks that have more than one (pf_merge_pieces), D / 4 lanes per
+// column, 4 head dims each.
 template <bool F16, int D>
 __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a) {
     using G = PfGeom<D>;
     constexpr int L = D / 4;  // lanes per column
-    static_assert(L % kPfMaxPieces == 0, "whole groups of one lane per piece");
     const int li = threadIdx.x % L;
     const int plane = blockIdx.y;
     const int b = plane / a.kv_heads, hk = plane % a.kv_heads;
@@ -892,39 +889,17 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a) {
     if (pieces <= 1) return;
     const int64_t rows = (int64_t)a.q_len * a.group;  // of a plane
     const int64_t step = rows * a.kv_heads * a.batch;
-    const int64_t row = plane * rows + col;
-    const int pl = li % kPfMaxPieces;
-    const float e = pl < pieces ? a.part_lse[row + pl * step] : -__builtin_inff();
-    float M = e;
-#pragma unroll
-    for (int o = 1; o < kPfMaxPieces; o <<= 1) M = fmaxf(M, __shfl_xor(M, o, kPfMaxPieces));
-    const float w = e == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(e - M);
-    float sum = w;
-#pragma unroll
-    for (int o = 1; o < kPfMaxPieces; o <<= 1) sum += __shfl_xor(sum, o, kPfMaxPieces);
-    const float *po = a.part_o + row * D + 4 * li;
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int p0 = 0; p0 < pieces; p0 += 4) {  // four pieces' rows in flight
-        f32x4 v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = *(const f32x4 *)(po + min(p0 + i, pieces - 1) * step * D);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float wp = __shfl(w, p0 + i, kPfMaxPieces);  // 0 past the last piece
-#pragma unroll
-            for (int k = 0; k < 4; ++k) acc[k] += wp > 0.0f ? wp * v[i][k] : 0.0f;
-        }
-    }
-    const float om = a.o_mul * (a.o_mul_dev ? a.o_mul_dev[0] : 1.0f);
-    const float inv = sum > 0.0f ? om / sum : 0.0f;
+    float o[4];
+    pf_merge_pieces<D>(a.part_o, a.part_lse, plane * rows + col, step, pieces, li,
+                       a.o_mul * (a.o_mul_dev ? a.o_mul_dev[0] : 1.0f), o);
     const int qi = (int)(col / a.group), g = (int)(col % a.group);
     u32x2 r;
     if constexpr (F16) {
-        r.x = pack_f16x2(acc[0] * inv, acc[1] * inv);
-        r.y = pack_f16x2(acc[2] * inv, acc[3] * inv);
+        r.x = pack_f16x2(o[0], o[1]);
+        r.y = pack_f16x2(o[2], o[3]);
     } else {
-        r.x = pack_bf16x2(acc[0] * inv, acc[1] * inv);
-        r.y = pack_bf16x2(acc[2] * inv, acc[3] * inv);
+        r.x = pack_bf16x2(o[0], o[1]);
+        r.y = pack_bf16x2(o[2], o[3]);
     }
     *(u32x2 *)(a.out + sq.o0 + (int64_t)qi * a.o_st + (int64_t)(hk * a.group + g) * a.o_sh + 4 * li) = r;
 }

@@ -481,11 +481,11 @@ __global__ __launch_bounds__(W * 64, W / 4) void prefill_f32_kernel(X3Args x, X3
     if (!ok) return;
     const float l = x3_sum_halves(st.l_run);
     const bool part = SPLIT && pieces > 1;
-    const float inv = l > 0.0f ? (part ? 1.0f : a.o_mul * (a.o_mul_dev ? a.o_mul_dev[0] : 1.0f)) / l : 0.0f;
+    const float inv = l == 0.0f ? 0.0f : (part ? 1.0f : a.o_mul * (a.o_mul_dev ? a.o_mul_dev[0] : 1.0f)) / l;
     float *orow;
     if (part) {
         const int64_t row = ((int64_t)piece * nplanes + plane) * ((int64_t)a.q_len * a.group) + c0 + 32 * wave + qr;
-        if (h == 0) a.part_lse[row] = l > 0.0f ? st.m_run + __builtin_log2f(l) : -__builtin_inff();
+        if (h == 0) a.part_lse[row] = pf_piece_lse(st.m_run, l);
         orow = a.part_o + row * D;
     } else {
         orow = (float *)a.out + sq.o0 + (int64_t)(q0 + qc) * a.o_st + (int64_t)head * a.o_sh;
@@ -519,34 +519,13 @@ __global__ __launch_bounds__(256) void prefill_f32_combine_kernel(X3Args x) {
     const int pieces = pf_pieces(n, x.piece_tiles, x.max_pieces);
     if (pieces <= 1) return;
     const int64_t rows = (int64_t)a.q_len * a.group, step = rows * a.kv_heads * a.batch;
-    const int64_t row = plane * rows + col;
-    const int pl = li % kPfMaxPieces;
-    const float e = pl < pieces ? a.part_lse[row + pl * step] : -__builtin_inff();
-    float M = e;
-#pragma unroll
-    for (int o = 1; o < kPfMaxPieces; o <<= 1) M = fmaxf(M, __shfl_xor(M, o, kPfMaxPieces));
-    const float w = e == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(e - M);
-    float sum = w;
-#pragma unroll
-    for (int o = 1; o < kPfMaxPieces; o <<= 1) sum += __shfl_xor(sum, o, kPfMaxPieces);
-    const float *po = a.part_o + row * D + 4 * li;
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int p0 = 0; p0 < pieces; p0 += 4) {
-        f32x4 v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = *(const f32x4 *)(po + min(p0 + i, pieces - 1) * step * D);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float wp = __shfl(w, p0 + i, kPfMaxPieces);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) acc[k] += wp > 0.0f ? wp * v[i][k] : 0.0f;
-        }
-    }
+    float r[4];
+    pf_merge_pieces<D>(a.part_o, a.part_lse, plane * rows + col, step, pieces, li,
+                       a.o_mul * (a.o_mul_dev ? a.o_mul_dev[0] : 1.0f), r);
     if (4 * li >= a.head_dim) return;
-    const float inv = sum > 0.0f ? a.o_mul * (a.o_mul_dev ? a.o_mul_dev[0] : 1.0f) / sum : 0.0f;
     const int qi = (int)(col / a.group), g = (int)(col % a.group);
     float *o = (float *)a.out + sq.o0 + (int64_t)qi * a.o_st + (int64_t)(hk * a.group + g) * a.o_sh + 4 * li;
-    *(f32x4 *)o = acc * inv;
+    *(f32x4 *)o = f32x4{r[0], r[1], r[2], r[3]};
 }
 
 // ---- host ----

@@ -9,6 +9,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "cqkv_device.h"
+
 namespace cqkv {
 
 // ceil(2^32 / group) for group 2 .. 32768, else 0: c / group of the columns of a workgroup
@@ -47,6 +49,51 @@ __host__ __device__ inline int pf_block_tiles(int q0, int q1, int lq, int lk, in
 }
 
 constexpr int kPfMaxPieces = 16;
+
+// log2-sum-exp of a piece's row from its running maximum and sum: -inf marks a row that sees no key
+// of the piece (l 0), and only that: a NaN sum (a NaN key or query, a score of +inf) stays NaN.
+__device__ inline float pf_piece_lse(float m, float l) {
+    return l == 0.0f ? -__builtin_inff() : m + __builtin_amdgcn_logf(l);
+}
+
+// Merges the pieces of one column's row: o = sum_p w_p o_p / sum_p w_p with w_p = 2^(lse_p - max lse)
+// (tq_combine_impl's formula, candle-core/kernels/turbo_quant_impl.h:659-685), times o_mul. Called by
+// the D / 4 lanes of a column, lane li with head dims 4 li .. 4 li + 3; row: the column's first
+// partial, step: rows of a piece. Lane p of each 16 loads piece p's lse (at most kPfMaxPieces = 16),
+// so the weights cost one load's latency. Pieces without a visible key are skipped; all others
+// count, also where the weight underflows or is NaN, so that non-finite rows come out as the unsplit
+// kernel's do.
+template <int D>
+__device__ inline void pf_merge_pieces(const float *part_o, const float *part_lse, int64_t row,
+                                       int64_t step, int pieces, int li, float o_mul, float *o) {
+    static_assert((D / 4) % kPfMaxPieces == 0, "whole groups of one lane per piece");
+    const int pl = li % kPfMaxPieces;
+    const float e = pl < pieces ? part_lse[row + pl * step] : -__builtin_inff();
+    float M = e;  // (NaN is passed over)
+#pragma unroll
+    for (int k = 1; k < kPfMaxPieces; k <<= 1) M = fmaxf(M, __shfl_xor(M, k, kPfMaxPieces));
+    const bool empty = e == -__builtin_inff();
+    const float w = empty ? -1.0f : __builtin_amdgcn_exp2f(e - M);  // -1: skipped
+    float sum = empty ? 0.0f : w;
+#pragma unroll
+    for (int k = 1; k < kPfMaxPieces; k <<= 1) sum += __shfl_xor(sum, k, kPfMaxPieces);
+    const float *po = part_o + row * D + 4 * li;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int p0 = 0; p0 < pieces; p0 += 4) {  // four pieces' rows in flight
+        f32x4 v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = *(const f32x4 *)(po + min(p0 + i, pieces - 1) * step * D);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float wp = __shfl(w, p0 + i, kPfMaxPieces);  // -1 past the last piece
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc[k] += wp < 0.0f ? 0.0f : wp * v[i][k];
+        }
+    }
+    const float inv = sum == 0.0f ? 0.0f : o_mul / sum;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) o[k] = acc[k] * inv;
+}
 
 // How a call's key ranges are split: column blocks of more than `tiles` key tiles in up to `pieces`
 // pieces (1: not at all), and the bytes of the partials.
