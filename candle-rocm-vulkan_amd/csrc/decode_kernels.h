@@ -794,18 +794,31 @@ __device__ inline void compute_tile(Tile<KF, VF, D> &cur, int tile, const Decode
     }
 }
 
-// Wavefronts per SIMD the register allocation must leave room for with MXFP4 keys and values:
-// 3 at D = 128 (168 VGPRs; at 176 only two fit and BASELINE config 3 runs 30 % slower), 4 at
-// D = 64; other formats, and D = 256 (one wavefront per SIMD, VGPRs and AGPRs), take what the
-// allocation gives.
-template <int KF, int VF, int D>
+// Wavefronts per SIMD the register allocation must leave room for; the kernels not named here take
+// what the allocation gives.
+//  * MXFP4 keys and values: 3 at D = 128 (168 VGPRs; at 176 only two fit and 64 ragged sequences of
+//    up to 32K tokens run 30 % slower), 4 at D = 64.
+//  * Left alone, the compiler lets the prologue's loads in flight (queries, then two tiles) cost the
+//    whole kernel a wavefront per SIMD where its registers are just below a limit, and the split
+//    counts assume the workgroups that fit without them. None of these spills with the floor: 4-bit
+//    keys and values at D = 256 (2; 268 to 312 registers without it), MXFP4 keys and MXFP8 values at
+//    D = 128 (3; 169), MXFP8 at D = 64 (4; 129). 8 x 32K tokens, 32 / 8 heads, D = 256: MXFP4 108.0 us
+//    per call without and 98.5 with the floor, TurboQuant-4 129.3 and 106.4, NVFP4 / TurboQuant-4 153
+//    and 121; 64 ragged sequences of up to 8K tokens, MXFP8, D = 64: 84.6 and 69.4.
+template <int KF, int VF, int D, bool TERMS, bool QS>
 constexpr int decode_min_waves() {
-    return KF == CQKV_FMT_MXFP4 && VF == CQKV_FMT_MXFP4 && D < 256 ? (D == 128 ? 3 : 4) : 1;
+    constexpr bool k4 = KF == CQKV_FMT_MXFP4 || KF == CQKV_FMT_NVFP4 || turbo_mse<KF>();
+    constexpr bool v4 = VF == CQKV_FMT_MXFP4 || turbo_mse<VF>();
+    if (KF == CQKV_FMT_MXFP4 && VF == CQKV_FMT_MXFP4 && D < 256) return D == 128 ? 3 : 4;
+    if (D == 256 && k4 && v4 && !QS) return 2;
+    if (KF == CQKV_FMT_MXFP4 && VF == CQKV_FMT_MXFP8 && D == 128 && !TERMS && !QS) return 3;
+    if (KF == CQKV_FMT_MXFP8 && VF == CQKV_FMT_MXFP8 && D == 64 && !TERMS && !QS) return 4;
+    return 1;
 }
 
 template <int KF, int VF, int D, int WAVES, bool TERMS, bool QS>
 __global__ __launch_bounds__(WAVES * 64)
-__attribute__((amdgpu_waves_per_eu(decode_min_waves<KF, VF, D>()))) void decode_kernel(DecodeArgs a) {
+__attribute__((amdgpu_waves_per_eu(decode_min_waves<KF, VF, D, TERMS, QS>()))) void decode_kernel(DecodeArgs a) {
     constexpr int NCH = D / 32;
     constexpr int NT = WAVES * 64;
     constexpr bool kTurbo =
@@ -814,8 +827,10 @@ __attribute__((amdgpu_waves_per_eu(decode_min_waves<KF, VF, D>()))) void decode_
     // TurboQuant code table (64 KB-aligned, see turbo_pair), which is live only during the tile
     // loop
     // (rows of D + 4 floats: with a row stride of a multiple of the banks, the 16 columns of one
-    // access met in the same banks)
-    constexpr int kRow = D + 4, kOWords = WAVES * 16 * kRow, kTabWords = kTurbo ? 256 * 64 : 0;
+    // access met in the same banks; rows of D where the 4 would push the compact tables below to
+    // 16 KB further on, 97 KB in all and one workgroup per CU instead of two)
+    constexpr int kRow = D + (D == 256 && kTurbo && (compact_tab<KF>() || compact_tab<VF>()) ? 0 : 4);
+    constexpr int kOWords = WAVES * 16 * kRow, kTabWords = kTurbo ? 256 * 64 : 0;
     __shared__ __attribute__((aligned(65536))) float sm_buf[kOWords > kTabWords ? kOWords : kTabWords];
     float(*sm_o)[16][kRow] = (float(*)[16][kRow])sm_buf;
     uint32_t *sm_tab = (uint32_t *)sm_buf;
