@@ -916,7 +916,12 @@ __attribute__((amdgpu_waves_per_eu(decode_min_waves<KF, VF, D, TERMS, QS>()))) v
     // wavefront are requested right behind them, so their latency passes behind the staging, the
     // rotation and the code tables, which with the merge at the end are most of the time where a
     // workgroup has few tiles (13 ragged sequences up to 3001 tokens, NVFP4: 22.0 -> 19.0 us for the
-    // kernel; 128K tokens of TurboQuant-4: 211.0 -> 205.8 us per call).
+    // kernel; 128K tokens of TurboQuant-4: 211.0 -> 205.8 us per call). The kernels that fill a SIMD
+    // with one wavefront (D = 256 without a floor in decode_min_waves) request the second tile after
+    // the operands are built: with both early the allocation moved tile registers through AGPRs in
+    // the loop (16 x 8K tokens, 32 / 8 heads, D = 256: FP8 93.2 us per call, 89.1 so, 89.4 with
+    // neither early; FP8 keys and NVFP4 values 109.7, 98.1 and 101.4; NVFP4 91.9, 86.4 and 96.0).
+    constexpr bool kBothEarly = D < 256 || decode_min_waves<KF, VF, D, TERMS, QS>() > 1;
     float(*sm_q)[kRow] = sm_o[0];
     Tile<KF, VF, D> ta, tb2;
     int t = tb + wave;
@@ -939,8 +944,10 @@ __attribute__((amdgpu_waves_per_eu(decode_min_waves<KF, VF, D, TERMS, QS>()))) v
         __builtin_amdgcn_sched_barrier(0);
         load_tile<KF, VF, D>(ta, t, t < te, lane, kr, ksr, vr, vsr, ktok_off, vtok_off);
         __builtin_amdgcn_sched_barrier(0);
-        load_tile<KF, VF, D>(tb2, t + WAVES, t + WAVES < te, lane, kr, ksr, vr, vsr, ktok_off, vtok_off);
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kBothEarly) {
+            load_tile<KF, VF, D>(tb2, t + WAVES, t + WAVES < te, lane, kr, ksr, vr, vsr, ktok_off, vtok_off);
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int k = 0; k < kIt; ++k) {
             const int c = c1 + kCols * k;
@@ -1065,6 +1072,10 @@ __attribute__((amdgpu_waves_per_eu(decode_min_waves<KF, VF, D, TERMS, QS>()))) v
 
     // Register sets A and B alternate; the scheduling barriers keep every load of one set
     // issued before the next set's, so each wait only covers the set about to be used.
+    if constexpr (!kBothEarly) {
+        load_tile<KF, VF, D>(tb2, t + WAVES, t + WAVES < te, lane, kr, ksr, vr, vsr, ktok_off, vtok_off);
+        __builtin_amdgcn_sched_barrier(0);
+    }
     for (; t < te; t += 2 * WAVES) {
         compute_tile<KF, VF, D, TERMS, QS>(ta, t, a, qhi, qlo, lane, lo, hi, lo_max, hi_min, Lb,
                                        koff, tab, m_run, l_run, acc, kProd ? qsop : qhi, ktab, vtab,
