@@ -155,8 +155,8 @@ size_t prefill_e4m3_workspace(int32_t batch, int32_t kv_len, int32_t kv_heads);
 // Plain-dtype attention (flash_plain.hip): argument checks, workspace, bytes per K / V element.
 int fa_plain_check(const char *who, int32_t dtype, int32_t kv_dtype, int32_t head_dim,
                    int64_t k_row_stride, int64_t v_row_stride, int64_t kv_len);
-size_t fa_plain_workspace_bytes(int32_t batch, int32_t q_len, int32_t kv_len, int32_t q_heads,
-                                int32_t kv_heads, int32_t head_dim, bool ragged);
+size_t fa_plain_workspace_bytes(int32_t dtype, int32_t batch, int32_t q_len, int32_t kv_len,
+                                int32_t q_heads, int32_t kv_heads, int32_t head_dim, bool ragged);
 int fa_kv_esz(int32_t kv_dtype);
 
 }  // namespace cqkv

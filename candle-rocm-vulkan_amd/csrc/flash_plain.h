@@ -681,8 +681,7 @@ __global__ __launch_bounds__(256) void fa_combine_kernel(FaArgs a) {
 
 // prefill_f32.hip: the f32-query call on split bf16 operands, where it takes it
 int prefill_f32_run(const FaArgs &f, const char *who, void *workspace, size_t workspace_bytes,
-                    hipStream_t st, bool *taken);
-size_t prefill_f32_workspace(int32_t batch, int32_t q_len, int32_t kv_len, int32_t q_heads,
-                             int32_t kv_heads, int32_t head_dim);
+                    size_t plain_bytes, hipStream_t st, bool *taken);
+size_t prefill_f32_workspace(const FaArgs &a);
 
 }  // namespace cqkv

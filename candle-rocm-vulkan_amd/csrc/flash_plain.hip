@@ -157,17 +157,17 @@ int fa_plain_run(FaArgs a, const char *who, void *workspace, size_t workspace_by
         a.q_vec = fa_vec_ok(a.q, qs, f32 ? 4 : 2) ? 1 : 0;
         a.o_vec = f32 && fa_vec_ok(a.out, os, 4) ? 1 : 0;
     }
+    size_t lse_off = 0;
+    const size_t need =
+        s > 1 ? fa_partials_bytes(s, (int64_t)a.batch * a.q_heads * a.q_len, dmax, &lse_off) : 0;
     if (f32) {
         bool taken;
-        const int rc = prefill_f32_run(a, who, workspace, workspace_bytes, st, &taken);
+        const int rc = prefill_f32_run(a, who, workspace, workspace_bytes, need, st, &taken);
         if (rc != CQKV_OK || taken) return rc;
     }
     void *ws = workspace;
     bool owned = false;
     if (s > 1) {
-        size_t lse_off;
-        const int64_t rows = (int64_t)a.batch * a.q_heads * a.q_len;
-        const size_t need = fa_partials_bytes(s, rows, dmax, &lse_off);
         if (ws && workspace_bytes < need)
             return fail(CQKV_ERR_WORKSPACE, "%s: workspace %zu < %zu bytes", who, workspace_bytes,
                         need);
@@ -188,14 +188,28 @@ int fa_plain_run(FaArgs a, const char *who, void *workspace, size_t workspace_by
     return CQKV_OK;
 }
 
-size_t fa_plain_workspace_bytes(int32_t batch, int32_t q_len, int32_t kv_len, int32_t q_heads,
-                                int32_t kv_heads, int32_t head_dim, bool ragged) {
+size_t fa_plain_workspace_bytes(int32_t dtype, int32_t batch, int32_t q_len, int32_t kv_len,
+                                int32_t q_heads, int32_t kv_heads, int32_t head_dim, bool ragged) {
     const int dmax = fa_dmax(head_dim);
     const FaPlan p = fa_plan(batch, kv_heads, (int64_t)q_len * (q_heads / kv_heads), kv_len, dmax,
                              ragged);
-    if (p.splits <= 1) return 0;
-    size_t lse_off;
-    return fa_partials_bytes(p.splits, (int64_t)batch * q_heads * q_len, dmax, &lse_off);
+    size_t lse_off, bytes = 0;
+    if (p.splits > 1) bytes = fa_partials_bytes(p.splits, (int64_t)batch * q_heads * q_len, dmax, &lse_off);
+    if (dtype == CQKV_F32) {
+        FaArgs a = {};
+        a.dtype = a.kv_dtype = CQKV_F32;
+        a.batch = batch;
+        a.q_len = q_len;
+        a.kv_len = kv_len;
+        a.q_heads = q_heads;
+        a.kv_heads = kv_heads;
+        a.group = q_heads / kv_heads;
+        a.head_dim = head_dim;
+        a.splits = p.splits;
+        a.tiles_per_split = p.tps;
+        bytes = std::max(bytes, prefill_f32_workspace(a));
+    }
+    return bytes;
 }
 
 // ---- paged: blocks of plain K / V ----

@@ -1137,15 +1137,13 @@ size_t flash_attn_workspace(int32_t dtype, int32_t batch, int32_t q_len, int32_t
         q_heads % kv_heads != 0 || head_dim <= 0 || head_dim > 256)
         return 0;
     const size_t plain =
-        fa_plain_workspace_bytes(batch, q_len, kv_len, q_heads, kv_heads, head_dim, varlen);
+        fa_plain_workspace_bytes(dtype, batch, q_len, kv_len, q_heads, kv_heads, head_dim, varlen);
     // a call of the MFMA prefill's shape whose q / out rows are not aligned for it runs the
     // plain kernel: size for either
     if (kv_len > 0 && pf_fast_path(dtype, head_dim, q_len))
         return std::max((pf_vt_bytes(batch, kv_len, kv_heads, head_dim) + 255) / 256 * 256 +
                             pf_part_bytes(head_dim, batch, q_len, kv_len, q_heads, kv_heads),
                         plain);
-    if (dtype == CQKV_F32)
-        return std::max(plain, prefill_f32_workspace(batch, q_len, kv_len, q_heads, kv_heads, head_dim));
     return plain;
 }
 

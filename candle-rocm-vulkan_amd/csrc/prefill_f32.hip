@@ -550,34 +550,73 @@ static size_t x3_images(const FaArgs &a) {
     return (size_t)a.batch * a.kv_heads * ((a.kv_len + kX3Bk - 1) / kX3Bk) * image;
 }
 
-// Whether a call's sizes take this path. Up to 64 columns per plane (one block of fa32_kernel), and
-// with more than 16 planes, which fill the chip by themselves, up to 127 (255 at D = 128), the images'
-// traffic and the blocks' padding cost more than the products gain (66 columns, 32 planes, 1000 keys,
-// D = 128: 44 us here, 38 us there; 142 columns, 48 planes, 653 keys: 71 and 63; 312 columns, 24
-// planes, 2780 keys: 155 and 153; 68 columns, 8 planes, 2000 keys: 39 and 42); below 96 keys a launch
-// more. The images are held to 2 GiB.
-static bool x3_sizes(const FaArgs &a) {
-    const int64_t cols = (int64_t)a.q_len * a.group, planes = (int64_t)a.batch * a.kv_heads;
-    const int64_t most = planes <= 16 ? 64 : a.head_dim <= 64 ? 127 : 255;  // columns left to fa32_kernel
-    return a.dtype == CQKV_F32 && a.head_dim <= 128 && a.head_dim % 8 == 0 && a.kv_len >= 96 &&
-           cols > most && planes <= 65535 && x3_images(a) <= ((size_t)2 << 30);
+// Key tiles (of bk keys) of a group of n columns, the mean over the groups of a plane (up to 32 of
+// them, evenly spaced) and the largest.
+static double x3_mean_tiles(const FaArgs &a, int wl, int wr, int n, int bk, int *most) {
+    const int64_t cols = (int64_t)a.q_len * a.group, groups = (cols + n - 1) / n, k = std::min<int64_t>(groups, 32);
+    double sum = 0.0;
+    *most = 0;
+    for (int64_t i = 0; i < k; ++i) {
+        const int64_t c0 = (k > 1 ? i * (groups - 1) / (k - 1) : 0) * n;
+        int begin;
+        const int t = pf_block_tiles((int)(c0 / a.group), (int)((std::min(c0 + n, cols) - 1) / a.group), a.q_len,
+                                     a.kv_len, wl, wr, bk, begin);
+        *most = std::max(*most, t);
+        sum += t;
+    }
+    return sum / k;
 }
 
-size_t prefill_f32_workspace(int32_t batch, int32_t q_len, int32_t kv_len, int32_t q_heads,
-                             int32_t kv_heads, int32_t head_dim) {
-    FaArgs a = {};
-    a.dtype = CQKV_F32;
-    a.batch = batch;
-    a.q_len = q_len;
-    a.kv_len = kv_len;
-    a.q_heads = q_heads;
-    a.kv_heads = kv_heads;
-    a.group = q_heads / kv_heads;
-    a.head_dim = head_dim;
-    if (!x3_sizes(a)) return 0;
+// Whether a call takes this path: where its estimate is 5 % below fa32_kernel's. Both are fitted to 800
+// calls of 17 to 1400 columns, 96 to 5000 keys, 1 to 96 planes, f32 and bf16 K / V, each measured on
+// both paths (the mean call is 0.6 % off the faster one; by column and plane counts alone, 14 %).
+//  * Here: the three launches, the plan's estimate (with more than two blocks per CU, the chip's rate),
+//    and the images written and the K / V read: within 10 % of the time of 90 % of the calls.
+//  * fa32_kernel: 1.5 us per 16-key tile of a wavefront's 16 columns (0.7 at D = 64), one wavefront a
+//    SIMD at a time, the longest split where the chip is not full, and the combine, a serial chain over
+//    the splits (0.4 us each) besides its traffic: within 15 %.
+// Short key ranges and few columns stay on fa32_kernel: 8 planes of 195 columns and 196 keys, D = 128:
+// 30.7 us here, 18.1 there; 16 planes of 300 columns and 300 keys: 33 and 21; up to 128 keys nothing was
+// faster here. 8 planes of 300 columns and 2780 keys: 73 and 53; 4 planes of 2800 columns and 2100 keys at
+// D = 64: 29 and 53.
+static bool x3_sizes(const FaArgs &a, int wl, int wr, const X3Plan &plan) {
+    const int64_t cols = (int64_t)a.q_len * a.group, planes = (int64_t)a.batch * a.kv_heads;
     const int dk = x3_dk(a.head_dim);
-    return (x3_images(a) + 255) / 256 * 256 +
-           std::max(x3_plan(dk, a, -1, 0).split.bytes, x3_plan(dk, a, -1, -1).split.bytes);
+    const bool d64 = dk == 64;
+    int most;
+    double us = plan.split.us;
+    if (us == 0.0)
+        us = (double)planes * ((cols + 255) / 256) / 256 * (d64 ? 2.5 : 4.9) *
+             (x3_mean_tiles(a, wl, wr, 256, kX3Bk, &most) + 2);
+    const double mb = (double)planes * a.kv_len * dk * 2 * (6 + fa_kv_esz(a.kv_dtype)) / 1e6;
+    const double here = d64 ? 8.5 + 1.12 * us + 0.15 * mb : 11.3 + 1.05 * us + 0.13 * mb;
+    const double per_simd = (double)planes * ((cols + 15) / 16) / 1024 * x3_mean_tiles(a, wl, wr, 16, 16, &most);
+    const double longest = (d64 ? 0.4 : 0.8) * std::min(most, 2 * a.tiles_per_split);
+    const double parts = a.splits > 1 ? (double)a.splits * cols * planes * dk * 8 / 8e6 : 0.0;
+    const double there = d64 ? 10.7 + 0.72 * std::max(per_simd, longest) + 0.40 * a.splits + 2.6 * parts
+                             : 8.4 + 1.49 * std::max(per_simd, longest) + 0.43 * a.splits + 2.9 * parts;
+    return here < 0.95 * there;
+}
+// What it can take at all.
+static bool x3_can(const FaArgs &a) {
+    return a.dtype == CQKV_F32 && a.head_dim <= 128 && a.head_dim % 8 == 0 && a.kv_len > 128 &&
+           (int64_t)a.q_len * a.group > 16 && (int64_t)a.batch * a.kv_heads <= 65535 &&
+           x3_images(a) <= ((size_t)2 << 30);
+}
+
+// a: sizes, dtypes and the splits that fa32_kernel would take; 0 where neither a causal nor a full mask
+// takes this path.
+size_t prefill_f32_workspace(const FaArgs &a) {
+    if (!x3_can(a)) return 0;
+    const int dk = x3_dk(a.head_dim);
+    size_t parts = 0;
+    bool any = false;
+    for (int wr = -1; wr <= 0; ++wr) {
+        const X3Plan p = x3_plan(dk, a, -1, wr);
+        any |= x3_sizes(a, -1, wr, p);
+        parts = std::max(parts, p.split.bytes);
+    }
+    return any ? (x3_images(a) + 255) / 256 * 256 + parts : 0;
 }
 
 template <int D, int W>
@@ -629,15 +668,18 @@ static void x3_launch(const X3Args &x, hipStream_t st) {
 }
 
 // Runs the call here when its sizes and alignment allow and the workspace (if any) holds it; *taken
-// says whether it did. (q / out rows 16-byte aligned; K / V rows are in whole 4-element pieces by
+// says whether it did. plain_bytes: the partials of fa32_kernel's plan. (q / out rows 16-byte aligned; K / V rows are in whole 4-element pieces by
 // fa_plain_run's check.)
 int prefill_f32_run(const FaArgs &f, const char *who, void *workspace, size_t workspace_bytes,
-                    hipStream_t st, bool *taken) {
+                    size_t plain_bytes, hipStream_t st, bool *taken) {
     *taken = false;
-    if (!x3_sizes(f) || !f.q_vec || !f.o_vec) return CQKV_OK;
+    if (!x3_can(f) || !f.q_vec || !f.o_vec) return CQKV_OK;
     const int dk = x3_dk(f.head_dim);
-    const size_t images = (x3_images(f) + 255) / 256 * 256;
     const X3Plan choice = x3_plan(dk, f, f.wl, f.wr);
+    const size_t images = (x3_images(f) + 255) / 256 * 256;
+    // (a workspace that holds the images but not the other kernel's partials serves the call here)
+    const bool only_here = workspace && workspace_bytes >= images && workspace_bytes < plain_bytes;
+    if (!only_here && !x3_sizes(f, f.wl, f.wr, choice)) return CQKV_OK;
     PfPlan plan = choice.split;
     if (workspace && workspace_bytes < images) return CQKV_OK;
     if (workspace && workspace_bytes < images + plan.bytes) plan = PfPlan{};

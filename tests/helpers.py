@@ -351,3 +351,14 @@ def gqa_attention_f64(q, k, v, scale):
 
 def relative_rms(got, exact) -> float:
     return float(np.sqrt(((got - exact) ** 2).sum() / (exact ** 2).sum()))
+
+
+def gpu_kernels(fn) -> set:
+    """Names of the kernels that fn() launches, without template arguments."""
+    from torch.profiler import ProfilerActivity, profile
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        fn()
+        torch.cuda.synchronize()
+    names = (e.name for e in p.events())
+    return {n.split("::")[1].split("<")[0].split("(")[0] for n in names if "cqkv::" in n}

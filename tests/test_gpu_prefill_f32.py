@@ -1,11 +1,15 @@
 """f32 queries on split bf16 operands (prefill_f32.hip): column and key remainders, the split of key
 ranges, both workgroup widths, masks, score terms, head dims below the padded ones, variable lengths
 and every K / V type, against float64 within the reference's f32 bar of 1e-5 of max |ref|; infinities;
-and the route of a call whose workspace or alignment does not serve the path."""
+and the route of a call whose workspace or alignment does not serve the path. Calls whose estimate is
+smaller on the f32 MFMA kernel (short key ranges, few columns) run there; the sizes marked so are
+checked to take the path."""
 import math
 
 import pytest
 import torch
+
+from tests.helpers import gpu_kernels
 
 pytestmark = pytest.mark.gpu
 
@@ -33,11 +37,16 @@ def attention_f64(q, k, v, scale, causal, wl=-1, softcap=0.0, alibi=None):
 
 
 def check(cq, dev, b, sq, sk, hq, hkv, d, kvd=torch.float32, causal=True, wl=-1, softcap=0.0,
-          alibi=None, scale=1.0):
+          alibi=None, scale=1.0, taken=None):
     q = randn(1, (b, sq, hq, d)) * scale
     k, v = randn(2, (b, sk, hkv, d), kvd), randn(3, (b, sk, hkv, d), kvd)
     got = cq.flash_attn(q.to(dev), k.to(dev), v.to(dev), 1 / math.sqrt(d), causal, window_left=wl,
                         softcap=softcap, alibi_slopes=None if alibi is None else alibi.to(dev))
+    if taken is not None:
+        names = gpu_kernels(lambda: cq.flash_attn(
+            q.to(dev), k.to(dev), v.to(dev), 1 / math.sqrt(d), causal, window_left=wl,
+            softcap=softcap, alibi_slopes=None if alibi is None else alibi.to(dev)))
+        assert ("prefill_f32_kernel" in names) == taken, names
     want = attention_f64(q, k, v, 1 / math.sqrt(d), causal, wl, softcap, alibi)
     assert (got.cpu().double() - want).abs().max() <= 1e-5 * want.abs().max()
 
@@ -47,6 +56,22 @@ def check(cq, dev, b, sq, sk, hq, hkv, d, kvd=torch.float32, causal=True, wl=-1,
 @pytest.mark.parametrize("sq,sk", [(129, 129), (86, 97), (257, 300), (65, 1000)])
 def test_column_and_key_remainders(cq, dev, d, hq, hkv, sq, sk):
     check(cq, dev, 1, sq, sk, hq, hkv, d)
+
+
+@pytest.mark.parametrize("d", [8, 64, 72, 128])
+@pytest.mark.parametrize("b,hq,hkv,sq,sk", [
+    (2, 6, 2, 129, 2500), (2, 6, 2, 257, 3001), (2, 6, 2, 513, 1111), (1, 16, 1, 86, 3001),
+    (1, 16, 1, 65, 4000), (1, 16, 1, 129, 1300), (8, 2, 2, 700, 705), (4, 2, 2, 1033, 1033),
+    (2, 2, 2, 383, 4000), (8, 2, 2, 511, 4000)])
+def test_remainders_on_the_path(cq, dev, d, b, hq, hkv, sq, sk):
+    check(cq, dev, b, sq, sk, hq, hkv, d, taken=True)
+
+
+@pytest.mark.parametrize("b,sq,sk,hq,hkv,d", [(1, 195, 196, 8, 8, 128), (2, 300, 300, 8, 8, 128),
+                                              (1, 40, 700, 32, 8, 128), (1, 20, 2000, 32, 2, 128),
+                                              (1, 300, 128, 16, 1, 64), (1, 4, 3000, 16, 4, 64)])
+def test_short_calls_stay_on_the_f32_mfma(cq, dev, b, sq, sk, hq, hkv, d):
+    check(cq, dev, b, sq, sk, hq, hkv, d, taken=False)
 
 
 @pytest.mark.parametrize("kvd", [torch.float32, torch.float16, torch.bfloat16])
@@ -66,14 +91,20 @@ def test_score_terms_and_large_scores(cq, dev):
     slopes = 0.05 * (1 + torch.arange(6, dtype=torch.float32))
     check(cq, dev, 1, 150, 400, 6, 2, 64, softcap=3.0, alibi=slopes)
     check(cq, dev, 1, 150, 400, 6, 2, 128, scale=20.0)
+    check(cq, dev, 2, 150, 2400, 6, 2, 64, softcap=3.0, alibi=slopes, taken=True)
+    check(cq, dev, 2, 150, 2400, 6, 2, 128, scale=20.0, taken=True)
 
 
-def test_variable_lengths_equal_f64(cq, dev):
-    lens = [200, 0, 1, 333, 64]
+@pytest.mark.parametrize("lens", [[200, 0, 1, 333, 64], [700, 0, 1, 1333, 640, 90]])
+def test_variable_lengths_equal_f64(cq, dev, lens):
     cu = torch.tensor([0, *torch.tensor(lens).cumsum(0)], dtype=torch.int32, device=dev)
     n, hq, hkv, d = sum(lens), 8, 2, 64
     q, k, v = randn(1, (n, hq, d)), randn(2, (n, hkv, d)), randn(3, (n, hkv, d))
-    got = cq.flash_attn_varlen(q.to(dev), k.to(dev), v.to(dev), cu, cu, 333, 333, 0.125, True).cpu()
+    got = cq.flash_attn_varlen(q.to(dev), k.to(dev), v.to(dev), cu, cu, max(lens), max(lens), 0.125,
+                               True).cpu()
+    if max(lens) > 1000:
+        assert "prefill_f32_kernel" in gpu_kernels(lambda: cq.flash_attn_varlen(
+            q.to(dev), k.to(dev), v.to(dev), cu, cu, max(lens), max(lens), 0.125, True))
     at = 0
     for m in lens:
         if m:
@@ -82,16 +113,20 @@ def test_variable_lengths_equal_f64(cq, dev):
         at += m
 
 
-def test_non_finite_inputs(cq, dev):
+@pytest.mark.parametrize("sq,sk", [(130, 200), (700, 2000)])
+def test_non_finite_inputs(cq, dev, sq, sk):
     """A key at -inf * sign(q) gives probability 0, an infinite value an infinite output; queries near
     the top of f32 keep their scores (no part overflows: their bf16 rounding would)."""
-    q = randn(1, (1, 130, 2, 64)).abs() + 0.5
-    k, v = randn(2, (1, 200, 2, 64)), randn(3, (1, 200, 2, 64))
+    q = randn(1, (1, sq, 2, 64)).abs() + 0.5
+    k, v = randn(2, (1, sk, 2, 64)), randn(3, (1, sk, 2, 64))
     k[0, 5] = -math.inf
     v[0, 9, 0, 3] = math.inf
     q[0, 100, 1, 5], k[0, :, 1, 5] = 3.4e38, k[0, :, 1, 5] * 2.0 ** -100
     got = cq.flash_attn(q.to(dev), k.to(dev), v.to(dev), 0.1, False).cpu()
-    keep = torch.arange(200) != 5
+    if sq > 130:
+        assert "prefill_f32_kernel" in gpu_kernels(
+            lambda: cq.flash_attn(q.to(dev), k.to(dev), v.to(dev), 0.1, False))
+    keep = torch.arange(sk) != 5
     want = attention_f64(q, k[:, keep], v[:, keep], 0.1, False)
     assert torch.isposinf(got[0, :, 0, 3]).all()
     fin = torch.isfinite(want)

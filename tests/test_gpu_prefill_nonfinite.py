@@ -7,9 +7,11 @@ import math
 import pytest
 import torch
 
+from tests.helpers import gpu_kernels
+
 pytestmark = pytest.mark.gpu
 
-SQ, SK, HQ, HKV, D = 40, 3000, 8, 2, 128
+SQ, SK, HQ, HKV, D = 70, 3000, 8, 2, 128
 UNSPLIT_BYTES = {  # V^T of the 16-bit kernel; the f32 kernel's images of 32-key tiles, three parts each
     torch.bfloat16: HKV * D * 3008 * 2, torch.float16: HKV * D * 3008 * 2,
     torch.float32: HKV * 94 * 6 * 2 * 32 * D}
@@ -32,6 +34,13 @@ def both(cq, dev, q, k, v, causal=True):
     split = cq.flash_attn(q, k, v, 0.09, causal, workspace=ws).float().cpu()
     whole = cq.flash_attn(q, k, v, 0.09, causal, workspace=ws[:few]).float().cpu()
     return split, whole
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_the_call_splits(cq, dev, dtype):
+    q, k, v = (x.to(dev) for x in inputs(dtype))
+    names = gpu_kernels(lambda: cq.flash_attn(q, k, v, 0.09, True))
+    assert ("prefill_f32_combine_kernel" if dtype == torch.float32 else "prefill_combine_kernel") in names
 
 
 def assert_same_kind(got, want, dtype):
