@@ -187,8 +187,14 @@ def _scratch(nbytes: int, device: torch.device) -> torch.Tensor | None:
     library launches on: the block goes back when the call returns and is reused in stream order.
     The library's own stream-ordered allocation costs the host 10 us per call, and its pool gives
     the memory back at every synchronization, so the next call waits 70 us for a new mapping
-    (a 300-token prefill chunk over 7000 keys, alone: 233 us, of which 157 us were kernels)."""
-    return torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
+    (a 300-token prefill chunk over 7000 keys, alone: 233 us, of which 157 us were kernels). Where
+    torch has no such block left the library allocates, and takes a path that needs less if need be."""
+    if not nbytes:
+        return None
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
 
 
 def _need_gpu(t: torch.Tensor, what: str) -> None:

@@ -24,6 +24,15 @@ int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
             return ::cqkv::fail(CQKV_ERR_HIP, "%s failed: %s", #expr, hipGetErrorString(e_)); \
     } while (0)
 
+// Stream-ordered scratch for a path that another can stand in for: null (no error) when there is
+// not enough memory.
+inline void *scratch_or_null(size_t bytes, hipStream_t st) {
+    void *p = nullptr;
+    if (hipMallocAsync(&p, bytes, st) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
 // Code bits per element, or 0 for an unknown format.
 inline int code_bits(int32_t format) {
     switch (format) {

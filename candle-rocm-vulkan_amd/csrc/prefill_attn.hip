@@ -1356,7 +1356,7 @@ int flash_attn_impl(const void *q, const int64_t q_strides[3], const void *k,
     void *vt = workspace;
     const size_t vt_bytes = pf_vt_bytes(batch, kv_len, kv_heads, head_dim);
     const size_t kst_off = (vt_bytes + 255) / 256 * 256;
-    size_t ws_bytes = e4m3 ? kst_off + pf_kst_bytes(batch, kv_len, kv_heads) : vt_bytes;
+    const size_t ws_bytes = e4m3 ? kst_off + pf_kst_bytes(batch, kv_len, kv_heads) : vt_bytes;
     if (workspace && workspace_bytes < ws_bytes)
         return fail(CQKV_ERR_WORKSPACE, "cqkv_flash_attn: workspace %zu < %zu bytes",
                     workspace_bytes, ws_bytes);
@@ -1364,11 +1364,14 @@ int flash_attn_impl(const void *q, const int64_t q_strides[3], const void *k,
     const size_t part_off = (ws_bytes + 255) / 256 * 256;
     PfPlan plan = pf_plan(pf_shape(head_dim), batch, q_len, kv_len, q_heads, kv_heads, window_left, window_right);
     if (plan.pieces > 1 && workspace && workspace_bytes < part_off + plan.bytes) plan = PfPlan{};
-    if (plan.pieces > 1) ws_bytes = part_off + plan.bytes;
+    const bool vt_owned = workspace == nullptr;
+    if (vt_owned && plan.pieces > 1) vt = scratch_or_null(part_off + plan.bytes, st);
+    if (!vt) {  // unsplit, or no memory for the partials
+        plan = PfPlan{};
+        CQKV_HIP_CHECK(hipMallocAsync(&vt, ws_bytes, st));
+    }
     a.piece_tiles = plan.tiles;
     a.max_pieces = plan.pieces;
-    const bool vt_owned = workspace == nullptr;
-    if (vt_owned) CQKV_HIP_CHECK(hipMallocAsync(&vt, ws_bytes, st));
     a.vt = (const uint16_t *)vt;
     if (plan.pieces > 1) {
         const size_t rows = (size_t)plan.pieces * batch * q_heads * q_len;

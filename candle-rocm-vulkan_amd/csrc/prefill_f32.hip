@@ -667,9 +667,9 @@ static void x3_launch(const X3Args &x, hipStream_t st) {
                        dim3(256), 0, st, x);
 }
 
-// Runs the call here when its sizes and alignment allow and the workspace (if any) holds it; *taken
-// says whether it did. plain_bytes: the partials of fa32_kernel's plan. (q / out rows 16-byte aligned; K / V rows are in whole 4-element pieces by
-// fa_plain_run's check.)
+// Runs the call here when its sizes and alignment allow and the workspace, or without one the free
+// memory, holds it; *taken says whether it did. plain_bytes: the partials of fa32_kernel's plan. (q /
+// out rows 16-byte aligned; K / V rows are in whole 4-element pieces by fa_plain_run's check.)
 int prefill_f32_run(const FaArgs &f, const char *who, void *workspace, size_t workspace_bytes,
                     size_t plain_bytes, hipStream_t st, bool *taken) {
     *taken = false;
@@ -693,7 +693,8 @@ int prefill_f32_run(const FaArgs &f, const char *who, void *workspace, size_t wo
     x.max_pieces = plan.pieces;
     x.group_m = pf_group_m(f.group);
     void *ws = workspace;
-    if (!ws) CQKV_HIP_CHECK(hipMallocAsync(&ws, images + plan.bytes, st));
+    if (!ws) ws = scratch_or_null(images + plan.bytes, st);
+    if (!ws) return CQKV_OK;  // no memory for the images: the other kernel needs none
     *taken = true;
     x.img = (uint8_t *)ws;
     if (plan.pieces > 1) {
