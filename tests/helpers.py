@@ -362,3 +362,9 @@ def gpu_kernels(fn) -> set:
         torch.cuda.synchronize()
     names = (e.name for e in p.events())
     return {n.split("::")[1].split("<")[0].split("(")[0] for n in names if "cqkv::" in n}
+
+
+def library_allocates(cq, monkeypatch):
+    """Calls without a workspace pass none, so the library takes its scratch from its stream-ordered
+    pool (the C ABI's null workspace); otherwise the front end gives it a block of torch's."""
+    monkeypatch.setattr(cq, "_scratch", lambda nbytes, device: None)

@@ -13,7 +13,7 @@ import pytest
 import torch
 
 from oracle import oracle as O
-from tests.helpers import assert_close_bf16
+from tests.helpers import assert_close_bf16, library_allocates
 
 pytestmark = pytest.mark.gpu
 
@@ -139,7 +139,7 @@ def test_unaligned_q_takes_plain_kernel(cq, dev):
     assert_close_bf16(got.float().cpu().numpy(), want)
 
 
-def test_explicit_workspace_matches_allocated(cq, dev):
+def test_explicit_workspace_matches_allocated(cq, dev, monkeypatch):
     b, sq, sk, hq, hkv, d = 2, 4, 3000, 8, 2, 128
     q = randn(81, (b, sq, hq, d), "f16").to(dev)
     k = randn(82, (b, sk, hkv, d), "f16").to(dev)
@@ -152,6 +152,13 @@ def test_explicit_workspace_matches_allocated(cq, dev):
     assert torch.equal(a, bb)
     with pytest.raises(cq.CqkvError):
         cq.flash_attn(q, k, v, 0.1, True, workspace=ws[:n // 2])
+    library_allocates(cq, monkeypatch)
+    assert torch.equal(a, cq.flash_attn(q, k, v, 0.1, True))
+    blocks = [(k.transpose(1, 2), v.transpose(1, 2), 2990), (k[:, :64].transpose(1, 2), v[:, :64].transpose(1, 2), 50)]
+    qb = q.transpose(1, 2).contiguous()
+    own = cq.flash_attn_blocks(qb, blocks, 0.1)
+    monkeypatch.undo()
+    assert torch.equal(own, cq.flash_attn_blocks(qb, blocks, 0.1))
 
 
 def test_refused_inputs(cq, dev):

@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from oracle import oracle as O
-from tests.helpers import assert_close_bf16
+from tests.helpers import assert_close_bf16, library_allocates
 
 pytestmark = pytest.mark.gpu
 
@@ -110,7 +110,7 @@ def test_flash_attn_fp8_decode_shape_and_float8_dtype(cq, dev):
 
 @pytest.mark.parametrize("d,dtype,sq", [(64, torch.bfloat16, 150), (256, torch.float16, 77),
                                          (96, torch.float16, 3), (128, torch.float16, 200)])
-def test_flash_attn_fp8_head_dims_f16_and_workspace(cq, dev, d, dtype, sq):
+def test_flash_attn_fp8_head_dims_f16_and_workspace(cq, dev, d, dtype, sq, monkeypatch):
     """The reference's FP8 K / V path takes every head dim of its tile kernels and f16 queries
     (flash_attn.rs:862-892; kernels fa_*_f16_f8 of flash_attn_impl.h): head dims 64 / 96 / 256,
     f16 queries and outputs, prefill and decode shapes; a caller workspace of
@@ -134,6 +134,8 @@ def test_flash_attn_fp8_head_dims_f16_and_workspace(cq, dev, d, dtype, sq):
     assert_close_bf16(out.float().cpu().numpy(), want)
     with pytest.raises(cq.CqkvError):
         cq.flash_attn_fp8_codes(qd, k8d, v8d, scale, True, kd, vd, workspace=ws[:n - 256])
+    library_allocates(cq, monkeypatch)
+    assert torch.equal(out, cq.flash_attn_fp8_codes(qd, k8d, v8d, scale, True, kd, vd))
 
 
 @pytest.mark.parametrize("d", [2, 8, 32, 64, 128, 256])

@@ -13,7 +13,7 @@ import pytest
 import torch
 
 from tests.helpers import (assert_close_bf16, assert_decode_parity, exact_decode, exact_scores,
-                           kv_source, oracle_decode, oracle_rows)
+                           kv_source, library_allocates, oracle_decode, oracle_rows)
 
 pytestmark = pytest.mark.gpu
 
@@ -105,7 +105,7 @@ def test_paged_single_segment(cq, dev, fmt):
     paged_case(cq, dev, fmt, 1, 8, 8, 64, [40], [64], seed=2)
 
 
-def test_paged_caller_workspace(cq, dev):
+def test_paged_caller_workspace(cq, dev, monkeypatch):
     """With a caller-sized workspace the call allocates nothing and gives the same result."""
     b, hq, hkv, d = 2, 8, 2, 128
     blocks = []
@@ -126,6 +126,13 @@ def test_paged_caller_workspace(cq, dev):
     assert torch.equal(a, c)
     with pytest.raises(cq.CqkvError):
         cq.decode_attention_paged(q, blocks, 0.1, workspace=ws[:16])
+    library_allocates(cq, monkeypatch)
+    assert torch.equal(a, cq.decode_attention_paged(q, blocks, 0.1))
+    cache = cq.TurboKvCache(cq.TURBO4, cq.TURBO4, b, hkv, d, 2000, device=dev)
+    cache.append(kv_source(7, (b, hkv, 2000, d)).to(dev), kv_source(8, (b, hkv, 2000, d)).to(dev))
+    own = cq.decode_attention(q, cache.k, cache.v, 2000, 0.1)
+    monkeypatch.undo()
+    assert torch.equal(own, cq.decode_attention(q, cache.k, cache.v, 2000, 0.1))
 
 
 def test_paged_decode_graph_capture_replays(cq, dev):

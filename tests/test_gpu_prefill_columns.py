@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from oracle import oracle as O
-from tests.helpers import assert_close_bf16
+from tests.helpers import assert_close_bf16, gpu_kernels, library_allocates
 
 pytestmark = pytest.mark.gpu
 
@@ -64,9 +64,10 @@ def test_split_key_ranges(cq, dev, d, hq, hkv, sq, sk, wl, wr):
     check(cq, dev, 1, sq, sk, hq, hkv, d, wl, wr)
 
 
-def test_split_in_a_callers_workspace(cq, dev):
-    """The queried workspace gives the allocating call's bits; one that holds V^T but not the
-    partials still serves the call, unsplit, within the bar."""
+def test_split_in_a_callers_workspace(cq, dev, monkeypatch):
+    """The queried workspace gives the bits of the call that allocates for itself, in the library as
+    from the front end; one that holds V^T but not the partials still serves the call, unsplit, within
+    the bar."""
     q, k, v = (randn(i, s).to(dev) for i, s in
                enumerate(((1, 64, 8, 128), (1, 4000, 2, 128), (1, 4000, 2, 128))))
     want = cq.flash_attn(q, k, v, 0.09, True)
@@ -77,6 +78,24 @@ def test_split_in_a_callers_workspace(cq, dev):
     assert n > vt
     got = cq.flash_attn(q, k, v, 0.09, True, workspace=ws[:vt])
     assert_close_bf16(got.float().cpu().numpy(), want.float().cpu().numpy())
+    library_allocates(cq, monkeypatch)
+    assert torch.equal(cq.flash_attn(q, k, v, 0.09, True), want)
+    assert "prefill_combine_kernel" in gpu_kernels(lambda: cq.flash_attn(q, k, v, 0.09, True))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_windowed_split_in_the_librarys_memory(cq, dev, dtype, monkeypatch):
+    """A window's plan is not one that the workspace query sizes for (causal and full): the library's
+    own allocation, sized by the call's plan, and the queried workspace both serve it."""
+    q, k, v = (randn(i, s).to(dev).to(dtype) for i, s in
+               enumerate(((2, 400, 8, 128), (2, 9000, 2, 128), (2, 9000, 2, 128))))
+    call = lambda: cq.flash_attn(q, k, v, 0.09, True, window_left=3000)
+    want = call()
+    library_allocates(cq, monkeypatch)
+    got = call()
+    assert {"prefill_combine_kernel", "prefill_f32_combine_kernel"} & gpu_kernels(call)
+    bar = 2e-2 if dtype == torch.bfloat16 else 1e-5
+    assert (got - want).abs().max() <= bar * want.abs().max()
 
 
 @pytest.mark.parametrize("d", [64, 128, 256])

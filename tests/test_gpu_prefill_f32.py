@@ -9,7 +9,7 @@ import math
 import pytest
 import torch
 
-from tests.helpers import gpu_kernels
+from tests.helpers import gpu_kernels, library_allocates
 
 pytestmark = pytest.mark.gpu
 
@@ -147,3 +147,24 @@ def test_workspaces_and_unaligned_rows(cq, dev):
     for got in (cq.flash_attn(q, k, v, 0.125, True, workspace=ws[:images]),
                 cq.flash_attn(odd, k, v, 0.125, True)):
         assert (got - want).abs().max() <= 1e-5 * want.abs().max()
+
+
+def test_workspaces_on_the_path(cq, dev, monkeypatch):
+    """A call that takes the path in the queried workspace, in the images alone (unsplit) and in the
+    library's own allocation."""
+    b, sq, sk, hq, hkv, d = 2, 257, 3001, 6, 2, 128
+    q, k, v = (randn(i, s).to(dev) for i, s in
+               enumerate(((b, sq, hq, d), (b, sk, hkv, d), (b, sk, hkv, d))))
+    call = lambda ws=None: cq.flash_attn(q, k, v, 0.125, True, workspace=ws)
+    want = call()
+    ws = torch.empty(cq.flash_attn_workspace_bytes(torch.float32, b, sq, sk, hq, hkv, d),
+                     dtype=torch.uint8, device=dev)
+    images = b * hkv * 94 * 6 * 2 * 32 * d
+    assert torch.equal(call(ws), want)
+    got = call(ws[:images])
+    assert (got - want).abs().max() <= 1e-5 * want.abs().max()
+    names = gpu_kernels(lambda: call(ws[:images]))
+    assert "prefill_f32_kernel" in names and "prefill_f32_combine_kernel" not in names
+    library_allocates(cq, monkeypatch)
+    assert torch.equal(call(), want)
+    assert "prefill_f32_combine_kernel" in gpu_kernels(call)
