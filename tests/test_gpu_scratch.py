@@ -72,14 +72,17 @@ def test_no_memory_left_for_the_scratch(cq, dev, dtype):
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
     total = torch.cuda.get_device_properties(dev).total_memory
+    taken = []
     try:
         torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(dev) + 1) / total, dev)
-        with pytest.raises(torch.OutOfMemoryError):
-            torch.empty(64 << 20, dtype=torch.uint8, device=dev)
+        with pytest.raises(torch.OutOfMemoryError):  # what earlier work left free in its segments
+            while True:
+                taken.append(torch.empty(16 << 20, dtype=torch.uint8, device=dev))
         cq.flash_attn(q, k, v, 0.09, True, out=out)
         torch.cuda.synchronize()
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0, dev)
+        del taken
     assert torch.equal(out, want)
 
 
