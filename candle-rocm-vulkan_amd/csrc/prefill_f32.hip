@@ -4,9 +4,11 @@
 //
 // Every f32 operand is the exact sum of three bf16 parts x = x0 + x1 + x2 (8 significant bits each,
 // rounded to nearest), so a product is x0 y0 + (x0 y1 + x1 y0) + (x0 y2 + x1 y1 + x2 y0) plus terms
-// below 2^-25 of it. The six products are exact on v_mfma_f32_32x32x16_bf16 and summed in f32, the
-// five small ones of a dot product in an accumulator of their own: fewer roundings than the f32 MFMA's
-// one per four terms, at 16 / 6 of its rate. Probabilities are f32 and split the same way.
+// below 2^-25 of it. The six products are exact on v_mfma_f32_32x32x16_bf16 and summed in f32: fewer
+// roundings than the f32 MFMA's one per four terms, at 16 / 6 of its rate. In K Q^T the five small ones
+// of a dot product come first in the one accumulator, so that the sums at full magnitude are one
+// rounding per 16 dims; in V^T P^T they have an accumulator per tile, added once. Probabilities are
+// f32 and split the same way.
 // 2048 causal tokens, 2 sequences, 12 / 4 heads, D = 128, call: 341 us in fa32_kernel's column mode (f32
 // MFMA, K / V read by every wavefront) -> 182 us; relative error against float64 4.9e-7 -> 3.1e-7. Equal
 // ranges (1024 x 4096, 64 heads) run at 216 TFLOP/s, 1.3 PFLOP/s of bf16 products, what a large bf16
@@ -19,9 +21,12 @@
 //    through LDS rings of three K and V^T stages (144 KB at D = 128) by asynchronous copies, one
 //    barrier per tile. With 96 products of 32 cycles a tile and wavefront against some 400 vector
 //    instructions and 48 operand reads, the matrix units are the bound.
-//  * Non-finite inputs: the whole value goes into part 2, whose only product is with the other
-//    side's part 0, so an infinity meets neither another infinity's remainder nor a zero part.
-//    Values below about 2^-110 lose their last parts (bf16 has f32's exponent range).
+//  * Non-finite queries and keys: the whole value goes into part 2, whose only product is with the
+//    other side's part 0, so an infinity meets neither another infinity's remainder nor a zero part.
+//    Non-finite V elements are zeros in the image, since a matrix product would carry them, times a
+//    zero probability, into all 32 columns of a tile; the rows that see their keys get them after the
+//    loop (x3_bad_values; nothing is done there where the wavefront's tiles hold none).
+//  * Inputs below about 2^-110 lose their last parts (bf16 has f32's exponent range).
 #include <algorithm>
 #include <utility>
 #include <vector>
@@ -56,6 +61,7 @@ __device__ inline int x3_swz_v(int d) { return (d >> 2) & 3; }
 struct X3Args {
     FaArgs f;
     uint8_t *img;     // (batch, kv head, tiles) images
+    uint32_t *bad;    // (batch, kv head, tiles): the tile's keys with a non-finite value (null: not kept)
     int32_t tiles;    // images per plane
     int32_t q_blocks;
     int32_t piece_tiles, max_pieces;
@@ -127,6 +133,7 @@ __global__ __launch_bounds__(256) void prefill_f32_stage_kernel(X3Args x) {
     const FaArgs &a = x.f;
     constexpr int CPR = D / 8, IT = kX3Bk * CPR / 256, ROW = D + 4;
     __shared__ __attribute__((aligned(16))) float vt[kX3Bk * ROW];
+    __shared__ uint32_t rows_bad[4 * IT];
     const int tile = blockIdx.x, plane = blockIdx.y;
     const int b = plane / a.kv_heads, hk = plane % a.kv_heads;
     const FaSeq sq = fa_sequence(a, b);
@@ -150,6 +157,23 @@ __global__ __launch_bounds__(256) void prefill_f32_stage_kernel(X3Args x) {
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
         const int id = threadIdx.x + 256 * i, row = id / CPR, c = id % CPR;
+        if (x.bad) {
+            bool any = false;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float v = vr[i][e >> 2][e & 3];
+                const bool fin = __builtin_fabsf(v) < __builtin_inff();
+                any |= !fin;
+                vr[i][e >> 2][e & 3] = fin ? v : 0.0f;
+            }
+            // this wavefront's 64 / CPR rows
+            const uint64_t lanes = __ballot(any);
+            uint32_t w = 0;
+#pragma unroll
+            for (int r = 0; r < 64 / CPR; ++r)
+                w |= (lanes >> (r * CPR) & ((1u << CPR) - 1) ? 1u : 0u) << r;
+            if ((threadIdx.x & 63) == 0) rows_bad[4 * i + (threadIdx.x >> 6)] = w << (row & 31);
+        }
         *(f32x4 *)&vt[row * ROW + 8 * c] = vr[i][0];
         *(f32x4 *)&vt[row * ROW + 8 * c + 4] = vr[i][1];
         uint32_t w[4][3];
@@ -162,6 +186,12 @@ __global__ __launch_bounds__(256) void prefill_f32_stage_kernel(X3Args x) {
                 u32x4{w[0][p], w[1][p], w[2][p], w[3][p]};
     }
     __syncthreads();
+    if (x.bad && threadIdx.x == 0) {
+        uint32_t w = 0;
+#pragma unroll
+        for (int i = 0; i < 4 * IT; ++i) w |= rows_bad[i];
+        x.bad[(int64_t)plane * x.tiles + tile] = w;
+    }
     // V^T: chunk j of row d holds keys 8j .. 8j+7 in the order of the S^T registers
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
@@ -313,6 +343,69 @@ __device__ __attribute__((always_inline)) inline void x3_pv(X3State<D> &st, cons
     }
 }
 
+// Non-finite V elements of the wavefront's n tiles from tile kt of the plane on: each is added to the rows that see its key, times the key's weight there, which only has to be zero
+// (0 times infinity is NaN, as in plain attention) or not.
+template <int D>
+__device__ __attribute__((always_inline)) inline void x3_bad_values(X3State<D> &st, const X3Args &x, int plane,
+                                                                    int kt, int n, int lane) {
+    const FaArgs &a = x.f;
+    const int h = lane >> 5, b = plane / a.kv_heads;
+    const int64_t tile0 = (int64_t)plane * x.tiles + kt;
+    const uint32_t *flags = x.bad + tile0;
+    const uint8_t *images = x.img + tile0 * x3_image<D>();
+    for (int i0 = 0; i0 < n; i0 += 64) {
+        const uint32_t m = i0 + lane < n ? flags[i0 + lane] : 0u;
+        for (uint64_t left = __ballot(m != 0); left; left &= left - 1) {
+            const int i = __builtin_ctzll(left);
+            for (uint32_t keys = __builtin_amdgcn_readlane(m, i); keys; keys &= keys - 1) {
+                const int r = __builtin_ctz(keys), key = (kt + i0 + i) * kX3Bk + r;
+                const uint8_t *kimg = images + (int64_t)(i0 + i) * x3_image<D>() + r * 2 * D;
+                float dot = 0.0f;
+#pragma unroll
+                for (int ks = 0; ks < D / 16; ++ks) {
+                    f32x4 ka[2] = {}, qa[2] = {};
+#pragma unroll
+                    for (int p = 2; p >= 0; --p) {
+                        asm volatile("" : "+v"(st.q[ks][p]));  // (or their sums are kept over the loop)
+                        const u32x4 w = *(const u32x4 *)(kimg + p * x3_part<D>() + (((2 * ks + h) ^ x3_swz_k<D>(r)) << 4));
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) {
+                            const int sh = e & 1;
+                            ka[e >> 2][e & 3] += __uint_as_float(sh ? w[e >> 1] & 0xffff0000u : w[e >> 1] << 16);
+                            qa[e >> 2][e & 3] += __uint_as_float(sh ? st.q[ks][p][e >> 1] & 0xffff0000u
+                                                                    : st.q[ks][p][e >> 1] << 16);
+                        }
+                    }
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) dot += ka[e >> 2][e & 3] * qa[e >> 2][e & 3];
+                    __builtin_amdgcn_sched_barrier(0);  // (few registers are left beside q and acc)
+                }
+                const float s = fa_logit2(x3_sum_halves(dot) * st.scale_log2, st.cap2, st.slope2, st.pos - key);
+                if (key >= st.qlo && key < st.qhi) {
+                    const float p = __builtin_amdgcn_exp2f(s + st.negm);
+                    const int64_t at = fa_sequence(a, b).v0 + (plane - b * a.kv_heads) * a.v_sh +
+                                       (int64_t)key * a.v_st + 4 * h;
+#pragma unroll
+                    for (int md = 0; md < D / 32; ++md)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const int d = 32 * md + 8 * j;
+                            if (d >= a.head_dim) continue;
+                            const f32x4 v = a.kv_dtype == CQKV_F32    ? x3_load4<CQKV_F32>(a.v, at + d)
+                                            : a.kv_dtype == CQKV_F16  ? x3_load4<CQKV_F16>(a.v, at + d)
+                                            : a.kv_dtype == CQKV_BF16 ? x3_load4<CQKV_BF16>(a.v, at + d)
+                                                                      : x3_load4<kKvE4M3>(a.v, at + d);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                                if (!(__builtin_fabsf(v[e]) < __builtin_inff())) st.acc[md][4 * j + e] += p * v[e];
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                }
+            }
+        }
+    }
+}
+
 #define X3_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt((((n) & 15) | (((n) >> 4) << 14)) | 0x0f70)
 
 // W wavefronts of 32 columns: 8 (two per SIMD), or 4 where blocks of 256 columns would leave CUs idle
@@ -368,6 +461,11 @@ __global__ __launch_bounds__(W * 64, W / 4) void prefill_f32_kernel(X3Args x, X3
                  a.wr, lo_last, hi);
     const int wtiles = wave_live ? min(max((hi + kX3Bk - 1) / kX3Bk - kt, 0), ntiles) : 0;
 
+    // whether its tiles hold non-finite values (x3_bad_values), read beside the queries
+    uint32_t bad = 0;
+    if (x.bad)
+        for (int i = lane; i < wtiles; i += 64) bad |= x.bad[(int64_t)plane * x.tiles + kt + i];
+
     X3State<D> st;
     const int c = cr0 + min(32 * wave + qr, ncol - 1);
     const int qc = pf_div_group(c, a.group, x.group_m), head = hk * a.group + (c - qc * a.group);
@@ -406,6 +504,7 @@ __global__ __launch_bounds__(W * 64, W / 4) void prefill_f32_kernel(X3Args x, X3
 
     const uint8_t *images = x.img + ((int64_t)plane * x.tiles + kt) * IMG;
     X3_WAIT_VMCNT(0);  // the loads above must not be counted by the copy waits below
+    const bool any_bad = __any(bad != 0);
     // Step t works on the scores of tile t and on P V of tile t - 1. The two wavefronts of a SIMD (w and
     // w + 4) order them so that one's softmax runs beside the other's products: the first takes P V
     // of tile t - 1, scores and softmax of tile t, the second the softmax and P V of tile t - 1, then the
@@ -477,6 +576,16 @@ __global__ __launch_bounds__(W * 64, W / 4) void prefill_f32_kernel(X3Args x, X3
 #undef X3_STEP
     X3_WAIT_VMCNT(0);
 
+    if (any_bad) {
+        // Values that were zeros in the images. Arguments and plane are read anew: kept over the loop they
+        // cost it registers (2 x 2048 causal tokens, 12 / 4 heads, D = 128: 162 us, 158.4 without this).
+        typedef const __attribute__((address_space(4))) X3Args kernarg_t;
+        uint64_t at = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+        uint32_t id = blockIdx.x;
+        asm volatile("" : "+s"(at), "+s"(id));
+        const X3Args &y = *(const X3Args *)(kernarg_t *)at;
+        x3_bad_values<D>(st, y, (int)(id % (uint32_t)(y.f.kv_heads * y.f.batch)), kt, wtiles, lane);
+    }
     // lane (qr, h): head dims 32 md + 8 (j / 4) + 4 h + j % 4 of column qr
     if (!ok) return;
     const float l = x3_sum_halves(st.l_run);
@@ -550,6 +659,12 @@ static size_t x3_images(const FaArgs &a) {
     return (size_t)a.batch * a.kv_heads * ((a.kv_len + kX3Bk - 1) / kX3Bk) * image;
 }
 
+// Bytes of the image region and of the flags behind it; the partials follow.
+static size_t x3_images_end(const FaArgs &a) { return (x3_images(a) + 255) / 256 * 256; }
+static size_t x3_flags(const FaArgs &a) {
+    return ((size_t)a.batch * a.kv_heads * ((a.kv_len + kX3Bk - 1) / kX3Bk) * 4 + 255) / 256 * 256;
+}
+
 // Key tiles (of bk keys) of a group of n columns, the mean over the groups of a plane (up to 32 of
 // them, evenly spaced) and the largest.
 static double x3_mean_tiles(const FaArgs &a, int wl, int wr, int n, int bk, int *most) {
@@ -616,7 +731,7 @@ size_t prefill_f32_workspace(const FaArgs &a) {
         any |= x3_sizes(a, -1, wr, p);
         parts = std::max(parts, p.split.bytes);
     }
-    return any ? (x3_images(a) + 255) / 256 * 256 + parts : 0;
+    return any ? x3_images_end(a) + x3_flags(a) + parts : 0;
 }
 
 template <int D, int W>
@@ -676,13 +791,13 @@ int prefill_f32_run(const FaArgs &f, const char *who, void *workspace, size_t wo
     if (!x3_can(f) || !f.q_vec || !f.o_vec) return CQKV_OK;
     const int dk = x3_dk(f.head_dim);
     const X3Plan choice = x3_plan(dk, f, f.wl, f.wr);
-    const size_t images = (x3_images(f) + 255) / 256 * 256;
+    const size_t images = x3_images_end(f), parts_off = images + x3_flags(f);
     // (a workspace that holds the images but not the other kernel's partials serves the call here)
     const bool only_here = workspace && workspace_bytes >= images && workspace_bytes < plain_bytes;
     if (!only_here && !x3_sizes(f, f.wl, f.wr, choice)) return CQKV_OK;
     PfPlan plan = choice.split;
     if (workspace && workspace_bytes < images) return CQKV_OK;
-    if (workspace && workspace_bytes < images + plan.bytes) plan = PfPlan{};
+    if (workspace && workspace_bytes < parts_off + plan.bytes) plan = PfPlan{};
     X3Args x = {};
     x.f = f;
     x.tiles = (f.kv_len + kX3Bk - 1) / kX3Bk;
@@ -693,13 +808,15 @@ int prefill_f32_run(const FaArgs &f, const char *who, void *workspace, size_t wo
     x.max_pieces = plan.pieces;
     x.group_m = pf_group_m(f.group);
     void *ws = workspace;
-    if (!ws) ws = scratch_or_null(images + plan.bytes, st);
+    if (!ws) ws = scratch_or_null(parts_off + plan.bytes, st);
     if (!ws) return CQKV_OK;  // no memory for the images: the other kernel needs none
     *taken = true;
     x.img = (uint8_t *)ws;
+    // (in the images alone, non-finite values stay in them and reach the other rows of their tiles)
+    if (!workspace || workspace_bytes >= parts_off) x.bad = (uint32_t *)((char *)ws + images);
     if (plan.pieces > 1) {
         const size_t rows = (size_t)plan.pieces * f.batch * f.q_heads * f.q_len;
-        x.f.part_o = (float *)((char *)ws + images);
+        x.f.part_o = (float *)((char *)ws + parts_off);
         x.f.part_lse = (float *)((char *)x.f.part_o + (rows * dk * 4 + 255) / 256 * 256);
     }
     if (dk == 64) choice.waves == 4 ? x3_launch<64, 4>(x, st) : x3_launch<64, 8>(x, st);

@@ -115,8 +115,9 @@ struct PfPlan {
 //    rows of 5 pieces).
 // A causal prompt of about as many blocks as CUs keeps them whole: its mean is half of its longest,
 // but the rate rises as CUs fall idle, and the partials cost what is left (2048 tokens, 32 / 8 heads:
-// 62.6 us whole, 66.2 us in halves; 3000 tokens: 91.7 and 110.2). No piece is under min_keys, so
-// shorter sequences are never split (512 keys in the 16-bit prefill).
+// 62.6 us whole, 66.2 us in halves; 3000 tokens: 91.7 and 110.2). Whole pieces have at least
+// min_keys (512 in the 16-bit prefill), so shorter key ranges are never split; the last piece of a block
+// may be anything above a quarter of a whole one (pf_pieces).
 struct PfShape {
     int nc, bk, head_dim;  // columns of a block, keys of a tile, head dim of the partials
     double lo, hi;         // step time, us: lo idle, lo + hi with every CU busy
@@ -125,7 +126,7 @@ struct PfShape {
 };
 inline PfPlan pf_plan(const PfShape &g, int batch, int q_len, int kv_len, int q_heads, int kv_heads,
                       int wl, int wr) {
-    constexpr int kCus = 256;
+    constexpr int kCus = 256;  // gfx950 (MI355X); a part with fewer would only be planned less well
     const int nc = g.nc, bk = g.bk, min_tiles = g.min_keys / bk, group = q_heads / kv_heads;
     const double lo = g.lo, hi = g.hi;
     const int64_t planes = (int64_t)batch * kv_heads, cols = (int64_t)q_len * group;

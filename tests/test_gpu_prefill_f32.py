@@ -1,6 +1,7 @@
 """f32 queries on split bf16 operands (prefill_f32.hip): column and key remainders, the split of key
 ranges, both workgroup widths, masks, score terms, head dims below the padded ones, variable lengths
-and every K / V type, against float64 within the reference's f32 bar of 1e-5 of max |ref|; infinities;
+and every K / V type, against float64 within the reference's f32 bar of 1e-5 of max |ref|; infinities
+and NaN, also in values of masked keys;
 and the route of a call whose workspace or alignment does not serve the path. Calls whose estimate is
 smaller on the f32 MFMA kernel (short key ranges, few columns) run there; the sizes marked so are
 checked to take the path."""
@@ -168,3 +169,29 @@ def test_workspaces_on_the_path(cq, dev, monkeypatch):
     library_allocates(cq, monkeypatch)
     assert torch.equal(call(), want)
     assert "prefill_f32_combine_kernel" in gpu_kernels(call)
+
+
+@pytest.mark.parametrize("kvd", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,sq,sk,hq,hkv,d,wl", [
+    (2, 700, 2000, 6, 2, 64, -1), (2, 257, 3001, 6, 2, 128, -1), (2, 600, 2500, 6, 2, 72, 500),
+    (1, 86, 3001, 16, 1, 128, -1), (8, 700, 705, 2, 2, 64, -1)])
+def test_bad_value_of_a_masked_key(cq, dev, kvd, b, sq, sk, hq, hkv, d, wl):
+    """Infinite and NaN values of keys that only some rows see: the other rows, some of them in the same
+    tile, have the bits of the call with zeros there; rows that see them show them in that head dim."""
+    q, k, v = (randn(i, s, t).to(dev) for i, s, t in
+               ((1, (b, sq, hq, d), torch.float32), (2, (b, sk, hkv, d), kvd), (3, (b, sk, hkv, d), kvd)))
+    bad = {sk - sq // 2: math.inf, sk - sq // 2 + 5: math.nan, sk - 1: -math.inf, sk - sq - 3: math.inf}
+    pos = torch.arange(sq) + sk - sq
+    clean = v.clone()
+    seen = {}
+    for i, (key, x) in enumerate(bad.items()):
+        v[0, key, 0, 7 * i], clean[0, key, 0, 7 * i] = x, 0.0
+        seen[7 * i] = (pos >= key) & ((pos - key <= wl) | (wl < 0))
+    call = lambda v: cq.flash_attn(q, k, v, 0.1, True, window_left=wl)
+    got, want = call(v).cpu(), call(clean).cpu()
+    assert "prefill_f32_kernel" in gpu_kernels(lambda: call(v))
+    for (key, x), (dim, s) in zip(bad.items(), seen.items()):
+        hit = got[0, s][:, :hq // hkv, dim]
+        assert hit.numel() and (hit.isnan() if math.isnan(x) else hit == x).all(), key
+        got[0, s, :hq // hkv, dim] = want[0, s, :hq // hkv, dim] = 0.0
+    assert torch.equal(got, want)

@@ -12,9 +12,10 @@ from tests.helpers import gpu_kernels
 pytestmark = pytest.mark.gpu
 
 SQ, SK, HQ, HKV, D = 70, 3000, 8, 2, 128
-UNSPLIT_BYTES = {  # V^T of the 16-bit kernel; the f32 kernel's images of 32-key tiles, three parts each
+# V^T of the 16-bit kernel; the f32 kernel's images of 32-key tiles, three parts each, and a word per tile
+UNSPLIT_BYTES = {
     torch.bfloat16: HKV * D * 3008 * 2, torch.float16: HKV * D * 3008 * 2,
-    torch.float32: HKV * 94 * 6 * 2 * 32 * D}
+    torch.float32: HKV * 94 * 6 * 2 * 32 * D + 768}
 DTYPES = [torch.bfloat16, torch.float16, torch.float32]
 
 
