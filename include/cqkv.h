@@ -358,7 +358,9 @@ int cqkv_flash_attn(const void *q, const int64_t q_strides[3], const void *k,
  * lengths, q_len / kv_len their maxima; dtype is q's, the K / V dtype does not change it): the
  * MFMA prefill's V^T copy, with the f32 partials of its split key ranges where few queries meet
  * many keys (a workspace that holds only V^T serves the call unsplit), or the plain kernel's split
- * partials (0 when it does not split). */
+ * partials (0 when it does not split). With f32 queries, where the split-bf16 path is the faster one:
+ * its tile images (12 bytes per K / V element pair, at most 2 GiB), flags and partials; a workspace
+ * that holds only the plain kernel's partials serves the call on that kernel. */
 size_t cqkv_flash_attn_workspace_bytes(int32_t dtype, int32_t batch, int32_t q_len,
                                        int32_t kv_len, int32_t q_heads, int32_t kv_heads,
                                        int32_t head_dim, int32_t varlen);
