@@ -29,7 +29,6 @@
 //  * Inputs below about 2^-110 lose their last parts (bf16 has f32's exponent range).
 #include <algorithm>
 #include <utility>
-#include <vector>
 
 #include "cqkv_device.h"
 #include "cqkv_host.h"
@@ -755,8 +754,9 @@ static void x3_launch(const X3Args &x, hipStream_t st) {
         return;
     }
     unsigned rows = (unsigned)(x.q_blocks * x.max_pieces);
-    if (!a.cu_q) {
-        std::vector<std::pair<int, int>> jobs;  // (-tiles, block << 4 | piece)
+    if (!a.cu_q && rows <= kPfMaxWgs) {
+        std::pair<int, int> jobs[kPfMaxWgs];  // (-tiles, block << 4 | piece)
+        unsigned count = 0;
         for (int qb = x.q_blocks - 1; qb >= 0; --qb) {
             const int64_t c0 = (int64_t)qb * x.nc, cols = (int64_t)a.q_len * a.group;
             int begin;
@@ -764,14 +764,14 @@ static void x3_launch(const X3Args &x, hipStream_t st) {
                                          a.q_len, a.kv_len, a.wl, a.wr, kX3Bk, begin);
             const int pieces = pf_pieces(n, x.piece_tiles, x.max_pieces);
             for (int p = 0; p < pieces; ++p)
-                jobs.push_back({p + 1 < pieces ? -x.piece_tiles : p * x.piece_tiles - n, qb << 4 | p});
+                jobs[count++] = {p + 1 < pieces ? -x.piece_tiles : p * x.piece_tiles - n, qb << 4 | p};
         }
-        if (jobs.size() <= kX3Jobs && x.q_blocks <= 4096) {
-            std::stable_sort(jobs.begin(), jobs.end(),
+        if (count <= kX3Jobs && x.q_blocks <= 4096) {
+            std::stable_sort(jobs, jobs + count,
                              [](const auto &l, const auto &r) { return l.first < r.first; });
-            for (size_t i = 0; i < jobs.size(); ++i) order.job[i] = (uint16_t)jobs[i].second;
-            order.n = (int)jobs.size();
-            rows = (unsigned)jobs.size();
+            for (unsigned i = 0; i < count; ++i) order.job[i] = (uint16_t)jobs[i].second;
+            order.n = (int)count;
+            rows = count;
         }
     }
     hipLaunchKernelGGL((prefill_f32_kernel<D, true, W>), dim3(rows * planes), dim3(W * 64), 0, st, x,

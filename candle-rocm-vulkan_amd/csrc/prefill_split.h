@@ -5,7 +5,6 @@
 #include <algorithm>
 #include <cstddef>
 #include <cstdint>
-#include <vector>
 
 #include <hip/hip_runtime.h>
 
@@ -124,16 +123,17 @@ struct PfShape {
     int setup, min_keys;   // tiles' worth of a workgroup's setup, smallest piece
     bool sorted;           // pieces are handed out by size: the CUs end together
 };
+constexpr int kCus = 256;  // gfx950 (MI355X); a part with fewer would only be planned less well
+constexpr int kPfMaxBlocks = 2 * kCus, kPfMaxWgs = 8 * kCus;  // planned (a plane's) and split into (a call's)
 inline PfPlan pf_plan(const PfShape &g, int batch, int q_len, int kv_len, int q_heads, int kv_heads,
                       int wl, int wr) {
-    constexpr int kCus = 256;  // gfx950 (MI355X); a part with fewer would only be planned less well
     const int nc = g.nc, bk = g.bk, min_tiles = g.min_keys / bk, group = q_heads / kv_heads;
     const double lo = g.lo, hi = g.hi;
     const int64_t planes = (int64_t)batch * kv_heads, cols = (int64_t)q_len * group;
     const int64_t blocks = (cols + nc - 1) / nc;
     PfPlan best;
-    if (planes * blocks > 2 * kCus || kv_len <= g.min_keys) return best;
-    std::vector<int> n(blocks);  // key tiles, in the order the blocks are handed out
+    if (planes * blocks > kPfMaxBlocks || kv_len <= g.min_keys) return best;
+    int n[kPfMaxBlocks];  // key tiles, in the order the blocks are handed out
     int most = 0;
     for (int64_t i = 0; i < blocks; ++i) {
         const int64_t c0 = (blocks - 1 - i) * nc;
@@ -145,7 +145,7 @@ inline PfPlan pf_plan(const PfShape &g, int batch, int q_len, int kv_len, int q_
     double &best_us = best.us;
     for (int p = 1; p <= kPfMaxPieces; ++p) {
         const int tiles = (most + p - 1) / p;
-        if (p > 1 && (tiles < min_tiles || planes * blocks * p > 8 * kCus)) break;
+        if (p > 1 && (tiles < min_tiles || planes * blocks * p > kPfMaxWgs)) break;
         int64_t wgs = 0, total = 0, split_cols = 0;
         int longest = 0;
         for (int64_t i = 0; i < blocks; ++i) {
