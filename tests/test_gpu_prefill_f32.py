@@ -195,3 +195,39 @@ def test_bad_value_of_a_masked_key(cq, dev, kvd, b, sq, sk, hq, hkv, d, wl):
         assert hit.numel() and (hit.isnan() if math.isnan(x) else hit == x).all(), key
         got[0, s, :hq // hkv, dim] = want[0, s, :hq // hkv, dim] = 0.0
     assert torch.equal(got, want)
+
+
+def test_bad_value_of_a_masked_key_elsewhere(cq, dev):
+    """The same in E4M3 codes (NaN), in the last batch and head, and in a variable-length batch whose
+    sequences start at other rows, with score terms."""
+    b, sq, sk, hq, hkv, d = 2, 257, 3001, 6, 2, 128
+    q, k, v = (randn(i, s).to(dev) for i, s in
+               enumerate(((b, sq, hq, d), (b, sk, hkv, d), (b, sk, hkv, d))))
+    k8, v8 = (x.to(torch.float8_e4m3fn).view(torch.uint8) for x in (k, v))
+    v8[1, sk - 100, 1, 77] = 0
+    want = cq.flash_attn_fp8_codes(q, k8, v8, 0.1, True, 0.5, 2.0).cpu()
+    v8[1, sk - 100, 1, 77] = 0x7f
+    call = lambda: cq.flash_attn_fp8_codes(q, k8, v8, 0.1, True, 0.5, 2.0)
+    got = call().cpu()
+    assert "prefill_f32_kernel" in gpu_kernels(call)
+    assert got[1, sq - 100:, 3:, 77].isnan().all()
+    got[1, sq - 100:, 3:, 77] = want[1, sq - 100:, 3:, 77] = 0.0
+    assert torch.equal(got, want)
+
+    lens = [700, 1, 1333, 640]
+    cu = torch.tensor([0, *torch.tensor(lens).cumsum(0)], dtype=torch.int32, device=dev)
+    n, d = sum(lens), 64
+    q, k, v = (randn(i, (n, h, d)).to(dev) for i, h in ((1, 8), (2, 2), (3, 2)))
+    slopes = (0.01 * torch.arange(1, 9, dtype=torch.float32)).to(dev)
+    call = lambda: cq.flash_attn_varlen(q, k, v, cu, cu, 1333, 1333, 0.125, True, softcap=20.0,
+                                        alibi_slopes=slopes)
+    at = 701 + 900
+    v[at, 1, 63] = 0.0
+    want = call().cpu()
+    v[at, 1, 63] = -math.inf
+    got = call().cpu()
+    assert "prefill_f32_kernel" in gpu_kernels(call)
+    hit = slice(at, 701 + 1333)
+    assert got[hit, 4:, 63].isneginf().all()
+    got[hit, 4:, 63] = want[hit, 4:, 63] = 0.0
+    assert torch.equal(got, want)
